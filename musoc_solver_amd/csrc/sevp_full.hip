@@ -24,6 +24,8 @@
 // only the independent element updates of one step run in parallel.
 #include <hip/hip_ext.h>
 
+#include <type_traits>
+
 #include "sevp_dev.h"
 #include "sevp_internal.h"
 #include "sevp_march.h"
@@ -229,17 +231,436 @@ hipError_t launch_resid(const ResidArgs &a, hipStream_t st) {
 }
 
 // ---------------------------------------------------------------------------
-// Sequential-order FP64 GEMM with fused epilogues.
-//   D(m, n) = sum_{k=0..K-1} A(m,k) * B(k,n)   (EP_NEGSUB: 0 - sum ... as
-//   successive subtractions)
-// One output per thread, so that the independent sequential chains fill the
-// GPU (a 64 x 1440 product has 92160 of them).  Tile 16 (m) x 16 (n), K in
-// chunks of 64 staged through LDS from a ring of register slots filled three
-// chunks ahead.
+// Sequential-order FP64 products: every output is one thread's sum over k
+// from zero, in order, with separately rounded multiply and add.
+
+// B's 16 values of a row of 16 lanes, one broadcast to the row: lane i of
+// each 16-lane row receives lane P's value (DPP row_newbcast).
+template <int P>
+__device__ __forceinline__ double row_bcast(double v) {
+  const long l = __double_as_longlong(v);
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(0L, l, 0x150 + P, 0xf, 0xf, true));
+}
+
+template <int I, int N, class F>
+__device__ __forceinline__ void unroll(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    unroll<I + 1, N>(f);
+  }
+}
+
+// The correction products of a solve, D(m, n) = sum_k A(m, k) B(k, n), both
+// operands with consecutive k adjacent (the error rows and a column-major
+// influence matrix), with fused epilogues.
+//
+// A computing wavefront holds 16 right-hand sides (the lanes of a row) by 4
+// columns (its four 16-lane rows), one sum a lane.  A lane's B values are its
+// column's, so a row of lanes holds 32 consecutive k of the column, two a
+// lane, and each k reaches the row by a DPP broadcast; only A is read from
+// LDS per term (16 bytes for two k).  An output and k cost 8 bytes of LDS
+// reads, half of what a tile that reads both operands from LDS costs, which
+// bounded such a kernel.  The multiply of a term does not depend on the sum:
+// the terms of the next 8 k are formed between the additions of these.  What
+// bounds it now is LDS all the same (97 to 109 bytes a clock and CU at 64
+// right-hand sides): 21 clocks a term; 64 right-hand sides at 960 columns
+// take 13.3 us (22.5 before), 32 at 1440 columns 17.7 us (32 before).
+//
+// A matrix comes from HBM once a solve, so a launch is that latency and its
+// sums.  NL loading wavefronts stream both operands into LDS with DMAs
+// (global_load_lds: no registers and no waits while they fly), R chunks of
+// 64 k ahead; a register ring of half that depth waited for HBM.  NW
+// computing wavefronts side by side share A's chunks.  One barrier a chunk,
+// in the middle of its sum, tells that the next chunk has landed and that the
+// one before is no longer read, so neither side waits at a chunk's start.
+// Past K both operands are zero in LDS: a sum that started from +0 keeps its
+// bits when +0 is added.
+constexpr int GS_K = 64;
+
+// 16 or 4 bytes a lane of a 64-lane run at dst (wave-uniform) come from src.
+__device__ __forceinline__ void load_lds16(const void *src, void *dst) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void *)(src),
+                                   (__attribute__((address_space(3))) void *)(dst), 16, 0, 0);
+}
+__device__ __forceinline__ void load_lds4(const void *src, void *dst) {
+  __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void *)(src),
+                                   (__attribute__((address_space(3))) void *)(dst), 4, 0, 0);
+}
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// The chunk barrier: the side that writes LDS waits for its writes; the side
+// that reads it has used what it read from the buffer that is written next,
+// and its reads in flight are of another.
+__device__ __forceinline__ void bar_written() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+__device__ __forceinline__ void bar_reader() { asm volatile("s_barrier" ::: "memory"); }
+
+// One workgroup's operand ring.  B: a computing wavefront's chunk is two
+// runs of 64 pairs in the order its lanes use them.  A: the rows of a pair
+// adjacent, so that the 16 rows' reads of one pair are one run.
+template <int NW, int R>
+struct SeqRing {
+  double2 b[R][NW][2][64];
+  double2 a[R][32][16];
+};
+
+// Loading wavefront `l` of NL: every NL-th of a chunk's DMAs.  W = 16: runs
+// of pairs at 16-byte boundaries (an even K; the clamped pairs past K are
+// whole pairs of the run).  W = 4: any boundary, each k clamped by itself.
+template <int NW, int NL, int R, int W>
+__device__ __forceinline__ void seq_load(const GemmArgs &p, SeqRing<NW, R> &S, int n0, int m0,
+                                         int rows, int nlast, int l, int lane) {
+  constexpr int PP = 16 / W;                             // DMAs of a run of 64 pairs
+  constexpr int I = (2 * NW + 8) * PP, PER = I / NL;  // DMAs of a chunk; of this wavefront
+  static_assert(I % NL == 0 && (R - 3) * PER <= 63, "the waits count this wavefront's DMAs");
+  const double *run[PER];
+  int off[PER];  // k of this lane's element in a chunk
+  char *dst[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int id = l + NL * i, blk = id / PP, e = (id % PP) * 64 + lane;  // element of the run
+    const int s = e / PP;                                                 // its pair's place
+    if (blk < 2 * NW) {
+      const int w = blk >> 1, q = blk & 1;
+      run[i] = p.b + (long)min(n0 + 4 * w + (s >> 4), p.N - 1) * p.b_sn;
+      off[i] = 32 * q + 2 * (s & 15);
+      dst[i] = reinterpret_cast<char *>(&S.b[0][w][q][0]) + (id % PP) * 64 * W;
+    } else {
+      const int ps = (blk - 2 * NW) * 64 + s;
+      run[i] = p.a + (long)(m0 + min(ps & 15, rows - 1)) * p.a_sm;
+      off[i] = 2 * (ps >> 4);
+      dst[i] = reinterpret_cast<char *>(&S.a[0][0][0]) + ((blk - 2 * NW) * 64 * PP + (id % PP) * 64) * W;
+    }
+  }
+  auto issue = [&](int c, int slot) {
+    const int k0 = c * GS_K;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int id = l + NL * i;
+      char *d = dst[i] + (long)slot * (id / PP < 2 * NW ? sizeof(S.b[0]) : sizeof(S.a[0]));
+      if constexpr (W == 16) {
+        load_lds16(run[i] + min(k0 + off[i], p.K - 2), d);
+      } else {
+        const int comp = lane & 3;
+        load_lds4(reinterpret_cast<const uint32_t *>(run[i] + min(k0 + off[i] + (comp >> 1), p.K - 1)) +
+                      (comp & 1), d);
+      }
+    }
+  };
+  // the chunks issued after the one waited for (at most R - 3) may still fly
+  auto landed = [&](int newer) {
+    unroll<0, R - 2>([&](auto N) {
+      constexpr int n = decltype(N)::value;
+      if (newer == n) wait_loads<n * PER>();
+    });
+  };
+  // zeros over what the last chunk's clamped addresses brought, past K
+  auto zero_past = [&](int c, int slot) {
+    if (c != nlast) return;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int id = l + NL * i;
+      char *d = dst[i] + (long)slot * (id / PP < 2 * NW ? sizeof(S.b[0]) : sizeof(S.a[0])) + lane * W;
+      const int k = c * GS_K + off[i];
+      if constexpr (W == 16) {
+        if (k >= p.K) *reinterpret_cast<double2 *>(d) = make_double2(0.0, 0.0);
+      } else {
+        if (k + ((lane & 3) >> 1) >= p.K) *reinterpret_cast<uint32_t *>(d) = 0u;
+      }
+    }
+  };
+  for (int c = 0; c < R && c <= nlast; ++c) issue(c, c);
+  landed(min(nlast, R - 3));
+  zero_past(0, 0);
+  bar_written();
+  int sn = 1;        // slot of chunk c + 1
+  int slot = R - 1;  // of chunk c - 1 + R
+  for (int c = 0; c < nlast; ++c) {
+    landed(min(nlast - c - 1, R - 3));
+    zero_past(c + 1, sn);
+    bar_written();
+    if (c >= 1 && c - 1 + R <= nlast) issue(c - 1 + R, slot);
+    slot = slot + 1 == R ? 0 : slot + 1;
+    sn = sn + 1 == R ? 0 : sn + 1;
+  }
+}
+
+template <int NW, int NL, int R, int W>
+__global__ __launch_bounds__(64 * (NW + NL)) void gemm_seq_kernel(GemmArgs p) {
+  constexpr int NT = 4 * NW;  // columns of the tile
+  __shared__ __align__(16) SeqRing<NW, R> S;
+  __shared__ double Ts[16][NT + 1];
+  span_begin(p.tspan);
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  // XCD-aware placement: the dispatcher deals workgroups to the 8 XCDs in
+  // turn, so the row tiles of one column tile get ids on the same XCD, one
+  // after another, and read that tile of B from HBM once (the others from
+  // the XCD's L2); ids past the last column tile have no tile
+  const int ntn = (p.N + NT - 1) / NT, nmb = (p.M + 15) / 16;
+  const int slot = blockIdx.x >> 3, tcol = (slot / nmb) * 8 + (blockIdx.x & 7);
+  if (tcol >= ntn) {
+    span_end(p.tspan);
+    return;
+  }
+  const int n0 = tcol * NT, m0 = (slot % nmb) * 16;
+  const int K = p.K, rows = min(16, p.M - m0);
+  const int nlast = (K + GS_K - 1) / GS_K - 1;  // the chunks before it are whole
+  if (wave >= NW) {
+    seq_load<NW, NL, R, W>(p, S, n0, m0, rows, nlast, wave - NW, lane);
+    __syncthreads();  // the computing wavefronts' sums are in Ts
+    span_end(p.tspan);
+    return;
+  }
+  // the epilogue's element (em, en) of this thread and its operands, which
+  // do not depend on the product (threads without one load the tile's first)
+  const bool eok = m0 + t / NT < p.M && n0 + t % NT < p.N;
+  const int em = eok ? m0 + t / NT : m0, en = eok ? n0 + t % NT : n0;
+  double xv = 0.0;
+  float cyv = 0.f;
+  double *ex = nullptr;
+  if (p.ep != EP_CPL) {
+    ex = p.x + (long)em * p.x_stride + f2(p.i2 + 2, en + 2, p.xrow);
+    xv = *ex;
+    if (p.g) cyv = p.cy[(long)en + (long)(p.cyrow - 1) * p.i2];
+  }
+  // A chunk's sum runs in eight groups of 8 k.  Before group g is added, A's
+  // values of group g + 2 are requested, and the products of group g + 1 are
+  // formed between its additions; the last two groups do so for the next
+  // chunk (slot sn).
+  const double2 *ab = &S.a[0][0][lane & 15];
+  const double2 *bb = &S.b[0][wave][0][lane];
+  double acc = 0.0, pr[2][8];
+  double2 av[2][4], bv[2], bn[2];
+  auto read_a = [&](int sl, auto G) {
+    constexpr int g = decltype(G)::value;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) av[g & 1][j] = ab[sl * (32 * 16) + (4 * g + j) * 16];
+  };
+  auto read_b = [&](int sl, double2 (&b_)[2]) {
+    const double2 *q = bb + sl * (sizeof(S.b[0]) / 16);
+    b_[0] = q[0];
+    b_[1] = q[64];
+  };
+  auto product = [&](const double2 (&b_)[2], auto G, auto J) {  // two terms of group g
+    constexpr int g = decltype(G)::value, j = decltype(J)::value, pi = (4 * g + j) & 15;
+    pr[g & 1][2 * j] = av[g & 1][j].x * row_bcast<pi>(b_[g / 4].x);
+    pr[g & 1][2 * j + 1] = av[g & 1][j].y * row_bcast<pi>(b_[g / 4].y);
+  };
+  // add group g; next: forms the two terms j of the group after it between
+  // the additions
+  auto add = [&](auto G, auto next) {
+    constexpr int g = decltype(G)::value;
+    unroll<0, 4>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      next(J);
+      acc = acc + pr[g & 1][2 * j];
+      acc = acc + pr[g & 1][2 * j + 1];
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  constexpr std::integral_constant<int, 0> g0{};
+  constexpr std::integral_constant<int, 1> g1{};
+  bar_reader();  // chunk 0 has landed
+  read_b(0, bv);
+  read_a(0, g0);
+  read_a(0, g1);
+  unroll<0, 4>([&](auto J) { product(bv, g0, J); });
+  int sl = 0;
+  for (int c = 0; c < nlast; ++c) {
+    const int sn = sl + 1 == R ? 0 : sl + 1;
+    unroll<0, 8>([&](auto G) {
+      constexpr int g = decltype(G)::value;
+      if constexpr (g == 4) bar_reader();
+      if constexpr (g == 5) read_b(sn, bn);
+      read_a(g + 2 < 8 ? sl : sn, std::integral_constant<int, (g + 2) & 7>{});
+      add(G, [&](auto J) {
+        if constexpr (g < 7) product(bv, std::integral_constant<int, (g + 1) & 7>{}, J);
+        else product(bn, g0, J);
+      });
+    });
+    bv[0] = bn[0];
+    bv[1] = bn[1];
+    sl = sn;
+  }
+  const int kc = K - nlast * GS_K;
+  unroll<0, 8>([&](auto G) {
+    constexpr int g = decltype(G)::value;
+    if (8 * g < kc) {
+      if constexpr (g + 2 < 8) read_a(sl, std::integral_constant<int, (g + 2) & 7>{});
+      add(G, [&](auto J) {
+        if constexpr (g < 7) product(bv, std::integral_constant<int, (g + 1) & 7>{}, J);
+      });
+    }
+  });
+  // through LDS to the epilogue's order, consecutive columns adjacent
+  Ts[lane & 15][4 * wave + (lane >> 4)] = acc;
+  __syncthreads();
+  if (eok) {
+    const double d = Ts[t / NT][t % NT];
+    switch (p.ep) {
+      case EP_FWD:
+        p.dum0[(long)em * p.dum0_stride + en] = xv;
+        *ex = xv - d;
+        break;
+      case EP_BWD:
+        *ex = xv + d;
+        p.out[(long)em * p.out_ld + en] = d;
+        if (p.g) p.g[(long)em * p.out_ld + en] = d * (double)cyv;
+        break;
+      default:  // EP_CPL
+        p.out[(long)em * p.out_ld + en] = d;
+        break;
+    }
+  }
+  span_end(p.tspan);
+}
+
+// The same products for few right-hand sides (M <= MR <= 8), where the kernel
+// above leaves most of its 16-row lanes idle and a launch lasts as long as
+// one sum: the products of a term are formed apart from the additions.  Two
+// wavefronts form them (a half wavefront takes one of the tile's four columns
+// and 64 k at a time, the loads of both operands R chunks ahead in
+// registers) and leave them in LDS; the third only adds, one sum a lane, at
+// the rate of an addition and its LDS read instead of the multiply's, the
+// broadcast's and the addition's (10 against 21 clocks a term: one right-hand
+// side at 720 columns takes 6.3 us, 9.5 in the kernel above, 17.4 before
+// both).  Products past K are +0, which keeps the bits of a sum that started
+// from +0.  Barriers as above: one a chunk, in the middle of its sum, with
+// three chunks in LDS.
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));  // at any 8-byte boundary
+
+template <int MR, int R>
+__global__ __launch_bounds__(192) void gemm_seq_few_kernel(GemmArgs p) {
+  __shared__ __align__(16) double P[3][4 * MR][GS_K + 2];
+  span_begin(p.tspan);
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int n0 = 4 * blockIdx.x, K = p.K;
+  const int nlast = (K + GS_K - 1) / GS_K - 1;
+  if (wave > 0) {
+    const int col = 2 * (wave - 1) + (lane >> 5), kp = 2 * (lane & 31);
+    const double *bcol = p.b + (long)min(n0 + col, p.N - 1) * p.b_sn;
+    d2u ra[R][MR], rb[R];
+    // a chunk past the last loads the last again: the waits count loads
+    auto fetch = [&](int c, d2u (&a_)[MR], d2u &b_) {
+      const int k = min(min(c, nlast) * GS_K + kp, K - 2);
+      b_ = *reinterpret_cast<const d2u *>(bcol + k);
+#pragma unroll
+      for (int m = 0; m < MR; ++m)
+        a_[m] = *reinterpret_cast<const d2u *>(p.a + (long)min(m, p.M - 1) * p.a_sm + k);
+    };
+#pragma unroll
+    for (int d = 0; d < R; ++d) fetch(d, ra[d], rb[d]);
+    int buf = 0;
+    for (int c0 = 0; c0 <= nlast; c0 += R) {
+      unroll<0, R>([&](auto D) {
+        constexpr int d = decltype(D)::value;
+        const int c = c0 + d;
+        if (c <= nlast) {
+          // past the end the pair came from K - 2: its second product is k = K - 1's
+          const int sh = c * GS_K + kp - (K - 2);
+#pragma unroll
+          for (int m = 0; m < MR; ++m) {
+            const double q0 = ra[d][m].x * rb[d].x, q1 = ra[d][m].y * rb[d].y;
+            *reinterpret_cast<double2 *>(&P[buf][4 * m + col][kp]) =
+                make_double2(sh <= 0 ? q0 : (sh == 1 ? q1 : 0.0), sh <= 0 ? q1 : 0.0);
+          }
+          fetch(c + R, ra[d], rb[d]);
+          bar_written();
+          buf = buf == 2 ? 0 : buf + 1;
+        }
+      });
+    }
+    if (p.tspan) __syncthreads();  // span_end's of the adding wavefront
+    return;
+  }
+  const int m = min(lane >> 2, p.M - 1), n = min(n0 + (lane & 3), p.N - 1);
+  const bool ok = (lane >> 2) < p.M && n0 + (lane & 3) < p.N;
+  double xv = 0.0;
+  float cyv = 0.f;
+  double *ex = nullptr;
+  if (p.ep != EP_CPL) {
+    ex = p.x + (long)m * p.x_stride + f2(p.i2 + 2, n + 2, p.xrow);
+    xv = *ex;
+    if (p.g) cyv = p.cy[(long)n + (long)(p.cyrow - 1) * p.i2];
+  }
+  const double *pl = &P[0][min(lane, 4 * MR - 1)][0];
+  constexpr int PB = sizeof(P[0]) / sizeof(double);
+  double acc = 0.0;
+  double2 v[4][4];
+  auto read = [&](const double *q, auto G) {
+    constexpr int g = decltype(G)::value;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[g & 3][j] = *reinterpret_cast<const double2 *>(q + 8 * g + 2 * j);
+  };
+  auto add = [&](auto G, auto then) {  // then: the read into the slots this group leaves
+    constexpr int g = decltype(G)::value;
+    double2 w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = v[g & 3][j];
+    then();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      acc = acc + w[j].x;
+      acc = acc + w[j].y;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // groups of 8 k, requested four groups ahead (an LDS read takes as long as
+  // two or three groups' additions); the second half of a chunk requests the
+  // next one's first half
+  const double *q = pl;
+  int buf = 0;
+  bar_reader();
+  unroll<0, 4>([&](auto G) { read(q, G); });
+  for (int c = 0; c < nlast; ++c) {
+    buf = buf == 2 ? 0 : buf + 1;
+    const double *qn = pl + buf * PB;
+    unroll<0, 8>([&](auto G) {
+      constexpr int g = decltype(G)::value;
+      if constexpr (g == 4) bar_reader();
+      add(G, [&] { read(g < 4 ? q : qn, std::integral_constant<int, (g + 4) & 7>{}); });
+    });
+    q = qn;
+  }
+  const int kc = K - nlast * GS_K;
+  unroll<0, 8>([&](auto G) {
+    constexpr int g = decltype(G)::value;
+    if (8 * g < kc)
+      add(G, [&] {
+        if constexpr (g < 4) read(q, std::integral_constant<int, (g + 4) & 7>{});
+      });
+  });
+  if (ok) {
+    switch (p.ep) {
+      case EP_FWD:
+        p.dum0[(long)m * p.dum0_stride + n] = xv;
+        *ex = xv - acc;
+        break;
+      case EP_BWD:
+        *ex = xv + acc;
+        p.out[(long)m * p.out_ld + n] = acc;
+        if (p.g) p.g[(long)m * p.out_ld + n] = acc * (double)cyv;
+        break;
+      default:  // EP_CPL
+        p.out[(long)m * p.out_ld + n] = acc;
+        break;
+    }
+  }
+  span_end(p.tspan);
+}
+
+// Square products of the influence build, D = A B (EP_COLMAJ) or
+// 0 - A B by successive subtractions (EP_NEGSUB): A and D with consecutive m
+// adjacent, B with consecutive k adjacent.  One output per thread, tile
+// 16 (m) x 16 (n), K in chunks of 64 staged through LDS.
 constexpr int GT_M = 16, GT_N = 16, GT_K = 64;
 
-__global__ __launch_bounds__(256) void gemm_seq_kernel(GemmArgs p) {
-  span_begin(p.tspan);
+__global__ __launch_bounds__(256) void gemm_square_kernel(GemmArgs p) {
   // both tiles k-contiguous (rows of GT_K + 2 doubles, 16-byte aligned) so a
   // thread reads two consecutive k of each operand with one 128-bit load
   __shared__ __align__(16) double As[GT_M][GT_K + 2];
@@ -252,7 +673,6 @@ __global__ __launch_bounds__(256) void gemm_seq_kernel(GemmArgs p) {
   const int ntn = (p.N + GT_N - 1) / GT_N, nmb = (p.M + GT_M - 1) / GT_M;
   const int slot = blockIdx.x >> 3, tcol = (slot / nmb) * 8 + (blockIdx.x & 7);
   if (tcol >= ntn) {
-    span_end(p.tspan);
     return;
   }
   const int n0 = tcol * GT_N, m0 = (slot % nmb) * GT_M;
@@ -385,33 +805,7 @@ __global__ __launch_bounds__(256) void gemm_seq_kernel(GemmArgs p) {
     }
   }
   const int n = n0 + tn, m = m0 + tm;
-  const int i0 = p.i2 + 2;
-  const double d = acc;
-  if (n < p.N && m < p.M) switch (p.ep) {
-    case EP_FWD: {
-      double *x = p.x + (long)m * p.x_stride;
-      const long xi = f2(i0, n + 2, p.xrow);
-      const double xv = x[xi];
-      p.dum0[(long)m * p.dum0_stride + n] = xv;
-      x[xi] = xv - d;
-      break;
-    }
-    case EP_BWD: {
-      double *x = p.x + (long)m * p.x_stride;
-      const long xi = f2(i0, n + 2, p.xrow);
-      x[xi] = x[xi] + d;
-      p.out[(long)m * p.out_ld + n] = d;
-      if (p.g) p.g[(long)m * p.out_ld + n] = d * (double)p.cy[(long)n + (long)(p.cyrow - 1) * p.i2];
-      break;
-    }
-    case EP_CPL:
-      p.out[(long)m * p.out_ld + n] = d;
-      break;
-    default:  // EP_NEGSUB, EP_COLMAJ: column-major output (m fastest)
-      p.out[(long)m + (long)n * p.out_ld] = d;
-      break;
-  }
-  span_end(p.tspan);
+  if (n < p.N && m < p.M) p.out[(long)m + (long)n * p.out_ld] = acc;
 }
 
 // T(i, k) = R(i, k) * CY(k, cyrow): columns of an n x n column-major matrix
@@ -431,14 +825,73 @@ hipError_t launch_scale_cols(const double *r, const float *cy, int cyrow, int i2
   return hipGetLastError();
 }
 
+// Computing wavefronts per workgroup of gemm_seq_kernel: as few as leave at
+// most one workgroup per CU, so that every CU streams a share of the matrix
+// and no CU runs two workgroups while another has none.
+static int gemm_seq_waves(const GemmArgs &a) {
+  const long nmb = (a.M + 15) / 16;
+  for (int nw : {1, 2, 4})
+    if (nmb * ((a.N + 4 * nw - 1) / (4 * nw)) <= 256) return nw;
+  return 8;
+}
+// Right-hand sides up to which the sums are added apart: 8 at 720 columns
+// take 8.7 us that way, 9.5 in gemm_seq_kernel, whose time is the same for
+// any count up to 16; past 8 the forming wavefronts would read more rows than
+// they can keep ahead.
+constexpr int GS_FEW = 8;
+
 long gemm_workgroups(const GemmArgs &a) {
-  return 8L * ((a.M + GT_M - 1) / GT_M) * (((a.N + GT_N - 1) / GT_N + 7) / 8);
+  if (a.ep == EP_NEGSUB || a.ep == EP_COLMAJ)
+    return 8L * ((a.M + GT_M - 1) / GT_M) * (((a.N + GT_N - 1) / GT_N + 7) / 8);
+  if (a.M <= GS_FEW) return (a.N + 3) / 4;
+  const int nt = 4 * gemm_seq_waves(a);
+  return 8L * ((a.M + 15) / 16) * (((a.N + nt - 1) / nt + 7) / 8);
+}
+
+template <int NW, int NL, int R, int W>
+static void gemm_seq_go(const GemmArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+  const dim3 grid((unsigned)gemm_workgroups(a)), block(64 * (NW + NL));
+  if (ev0) hipExtLaunchKernelGGL((gemm_seq_kernel<NW, NL, R, W>), grid, block, 0, st, ev0, ev1, 0, a);
+  else hipLaunchKernelGGL((gemm_seq_kernel<NW, NL, R, W>), grid, block, 0, st, a);
+}
+
+template <int MR, int R>
+static void gemm_few_go(const GemmArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+  const dim3 grid((unsigned)gemm_workgroups(a)), block(192);
+  if (ev0) hipExtLaunchKernelGGL((gemm_seq_few_kernel<MR, R>), grid, block, 0, st, ev0, ev1, 0, a);
+  else hipLaunchKernelGGL((gemm_seq_few_kernel<MR, R>), grid, block, 0, st, a);
 }
 
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-  const dim3 grid((unsigned)gemm_workgroups(a));
-  if (ev0) hipExtLaunchKernelGGL(gemm_seq_kernel, grid, dim3(256), 0, st, ev0, ev1, 0, a);
-  else hipLaunchKernelGGL(gemm_seq_kernel, grid, dim3(256), 0, st, a);
+  if (a.M < 1 || a.N < 1 || a.K < 1) return hipErrorInvalidValue;
+  if (a.ep == EP_NEGSUB || a.ep == EP_COLMAJ) {
+    if (a.a_sm != 1 || a.b_sk != 1) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(gemm_square_kernel, dim3((unsigned)gemm_workgroups(a)), dim3(256), 0, st, a);
+    return hipGetLastError();
+  }
+  if (a.a_sk != 1 || a.b_sk != 1 || a.K < 2) return hipErrorInvalidValue;
+  if (a.M <= GS_FEW) {
+    if (a.M == 1) gemm_few_go<1, 12>(a, st, ev0, ev1);
+    else if (a.M == 2) gemm_few_go<2, 8>(a, st, ev0, ev1);
+    else if (a.M <= 4) gemm_few_go<4, 8>(a, st, ev0, ev1);
+    else gemm_few_go<8, 5>(a, st, ev0, ev1);
+    return hipGetLastError();
+  }
+  const int nw = gemm_seq_waves(a);
+  // 16-byte DMAs need every run of k at a 16-byte boundary
+  const bool w16 = a.K % 2 == 0 && a.a_sm % 2 == 0 && a.b_sn % 2 == 0 &&
+                   ((uintptr_t)a.a & 15) == 0 && ((uintptr_t)a.b & 15) == 0;
+  if (w16) {
+    if (nw == 1) gemm_seq_go<1, 2, 8, 16>(a, st, ev0, ev1);
+    else if (nw == 2) gemm_seq_go<2, 2, 6, 16>(a, st, ev0, ev1);
+    else if (nw == 4) gemm_seq_go<4, 2, 6, 16>(a, st, ev0, ev1);
+    else gemm_seq_go<8, 2, 6, 16>(a, st, ev0, ev1);
+  } else {
+    if (nw == 1) gemm_seq_go<1, 4, 8, 4>(a, st, ev0, ev1);
+    else if (nw == 2) gemm_seq_go<2, 4, 6, 4>(a, st, ev0, ev1);
+    else if (nw == 4) gemm_seq_go<4, 4, 6, 4>(a, st, ev0, ev1);
+    else gemm_seq_go<8, 8, 6, 4>(a, st, ev0, ev1);
+  }
   return hipGetLastError();
 }
 
