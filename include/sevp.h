@@ -202,7 +202,7 @@ int sevp_matinv(double *b, int n);
  * hipMalloc).  The result is bitwise sevp_matinv's.  b_dev: n x n FP64
  * column-major, device.  zero_pivots_dev (device int, may be NULL) receives
  * the zero pivots met.  Enqueued on hip_stream (NULL: the null stream); the
- * call does not wait.  The inversion's scratch is a fixed 2 MiB device array
+ * call does not wait.  The inversion's scratch is a fixed 4 MiB device array
  * per GPU (orders up to 4096; larger ones are refused with SEVP_E_ARG),
  * shared by every call on that GPU: calls that overlap in time on one GPU
  * race. */

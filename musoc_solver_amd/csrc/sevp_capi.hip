@@ -2896,8 +2896,8 @@ extern "C" int sevp_matinv(double *b, int n) {
 // GPU share the array: calls that overlap in time on one GPU race.
 namespace {
 constexpr int kNoAllocMaxN = 4096;
-constexpr size_t kNoAllocCounter = 2 * 32 * (size_t)kNoAllocMaxN;  // counter slot (in doubles)
-constexpr size_t kNoAllocDoubles = kNoAllocCounter + 32;           // 2 MiB + 256 B
+constexpr size_t kNoAllocCounter = 4 * 32 * (size_t)kNoAllocMaxN;  // counter slot (in doubles)
+constexpr size_t kNoAllocDoubles = kNoAllocCounter + 32;           // 4 MiB + 256 B
 constexpr int kNoAllocDevices = 64;
 std::mutex g_noalloc_mu;
 double *g_noalloc_ptr[kNoAllocDevices] = {};

@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define SEVP_WAVE 64
 
 // Column-major (Fortran) 2-D index with 1-based i, j.
@@ -54,6 +56,30 @@ __device__ __forceinline__ double wave_shl1_zero(double v) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x130, 0xf, 0xf, true);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x130, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
+}
+
+// Lane i of each 16-lane row receives the row's lane P (DPP row_newbcast).
+template <int P>
+__device__ __forceinline__ double row_bcast(double v) {
+  const long l = __double_as_longlong(v);
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(0L, l, 0x150 + P, 0xf, 0xf, true));
+}
+
+// Lane i of each quad receives the quad's lane P (DPP quad_perm).
+template <int P>
+__device__ __forceinline__ double quad_bcast(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x55 * P, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x55 * P, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// f(I), f(I + 1), ... f(N - 1) with constant arguments.
+template <int I, int N, class F>
+__device__ __forceinline__ void unroll(F f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    unroll<I + 1, N>(f);
+  }
 }
 
 // Broadcast lane `src` (wave-uniform) of a double.

@@ -24,8 +24,6 @@
 // only the independent element updates of one step run in parallel.
 #include <hip/hip_ext.h>
 
-#include <type_traits>
-
 #include "sevp_dev.h"
 #include "sevp_internal.h"
 #include "sevp_march.h"
@@ -233,22 +231,6 @@ hipError_t launch_resid(const ResidArgs &a, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // Sequential-order FP64 products: every output is one thread's sum over k
 // from zero, in order, with separately rounded multiply and add.
-
-// B's 16 values of a row of 16 lanes, one broadcast to the row: lane i of
-// each 16-lane row receives lane P's value (DPP row_newbcast).
-template <int P>
-__device__ __forceinline__ double row_bcast(double v) {
-  const long l = __double_as_longlong(v);
-  return __longlong_as_double(__builtin_amdgcn_update_dpp(0L, l, 0x150 + P, 0xf, 0xf, true));
-}
-
-template <int I, int N, class F>
-__device__ __forceinline__ void unroll(F f) {
-  if constexpr (I < N) {
-    f(std::integral_constant<int, I>{});
-    unroll<I + 1, N>(f);
-  }
-}
 
 // The correction products of a solve, D(m, n) = sum_k A(m, k) B(k, n), both
 // operands with consecutive k adjacent (the error rows and a column-major
