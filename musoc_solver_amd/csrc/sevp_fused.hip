@@ -152,11 +152,12 @@ __device__ __forceinline__ void part_tile(const typename KT::A *alt, int mb0, in
 #pragma unroll
   for (int mb = 0; mb < MBW; ++mb) ab[mb] = alt + ((long)min(mb0 + mb, mtiles - 1) * nchk * 64 + lane) * 4;
   const int clast = max(c_hi - 1, 0);
-  auto group = [&](int c0) {
-    AV av[G][MBW];
-    BV bv[G];
+  auto group = [&](auto size, int c0) {
+    constexpr int C = decltype(size)::value;
+    AV av[C][MBW];
+    BV bv[C];
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
+    for (int g = 0; g < C; ++g) {
       const long ch = min(c0 + g, clast);
       bv[g] = *reinterpret_cast<const BV *>(bb + ch * 256);
 #pragma unroll
@@ -167,20 +168,34 @@ __device__ __forceinline__ void part_tile(const typename KT::A *alt, int mb0, in
     // many registers for that: the compiler interleaves them)
     if constexpr (!std::is_same<KT, KF64>::value) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+    for (int g = 0; g < C; ++g)
       if (c0 + g < c_hi)
 #pragma unroll
         for (int mb = 0; mb < MBW; ++mb) acc[mb] = KT::mma(av[g][mb], bv[g], acc[mb]);
   };
+  // A share that a smaller group holds takes that one: a load past the share
+  // is a repeated one, but a compute unit takes 64 bytes a clock either way (one
+  // right-hand side, 720 columns, FP64: 3.52 ms a solve with twelve chunks for
+  // each wavefront's six, 3.37 without; FP32, 8 wavefronts, 400 columns, 8: 3.26
+  // and 2.77; 800, 24: 8.84 and 8.30).  Not where the registers are full with
+  // the whole group's: FP32 in 16 wavefronts.
+  if constexpr (G == 12 || (G == 6 && MBW == 1) || std::is_same<KT, KF64>::value) {
+    typedef std::integral_constant<int, (G + 1) / 2> Half;
+    typedef std::integral_constant<int, (G + 3) / 4> Quarter;
+    const int share = c_hi - c_lo;
+    if (share <= Quarter::value) return group(Quarter{}, c_lo);
+    if (share <= Half::value) return group(Half{}, c_lo);
+  }
+  typedef std::integral_constant<int, G> Whole;
   // the first group outside the loop: straight-line code, so its loads
   // follow the caller's earlier loads without waiting for them (the FP64
   // operands keep the plain loop, which needs fewer registers)
   int c0 = c_lo;
   if constexpr (!std::is_same<KT, KF64>::value) {
-    group(c0);
+    group(Whole{}, c0);
     c0 += G;
   }
-  for (; c0 < c_hi; c0 += G) group(c0);
+  for (; c0 < c_hi; c0 += G) group(Whole{}, c0);
 }
 
 // The product tile of a workgroup: W wavefronts, each its share of the K
@@ -207,6 +222,8 @@ __device__ __forceinline__ double product_tile(const typename KT::A *alt, int mb
   for (int mb = 0; mb < MBW; ++mb)
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[(wave * MBW + mb) * 256 + KT::row(q, i) * 16 + (lane & 15)] = acc[mb][i];
+  if constexpr (std::is_same<KT, KF64>::value)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the epilogue's operands (Operands) too
   __syncthreads();
   double s = 0.0;
   if (threadIdx.x < 256 * MBW)
@@ -234,88 +251,203 @@ __device__ __forceinline__ const FT *rhs_ptr(const float *f, const double *f64) 
   else return f;
 }
 
+// FP64: the epilogue's operands that do not depend on the product, fetched
+// before it into LDS by DMA, so that they are on their way with the product's
+// operands, which take the registers, and there when the product is (720
+// columns, one right-hand side: 3.37 ms a solve with them loaded behind the
+// product, 3.16 with these; 800 columns, 24: 3.83 and 3.71).  FP32 and BF16
+// launches are slower with these than with registers (8 wavefronts: 8.51 ms
+// against 8.35 at 800 columns) or without (16: 35.9 against 35.2 at 1440 x 720
+// with 64), their product's loads waiting behind them in every wavefront.
+//
+// Output t of the workgroup has dword k at op[k][t]; the wavefronts share the
+// dwords out (those of 256 MBW outputs each, every NS-th), all at the addresses
+// of output threadIdx.x % (256 MBW), so an address is valid for every thread.
+template <int W, int MBW, int N>
+struct Operands {
+  static constexpr int T = 256 * MBW, NS = W / (4 * MBW);
+  uint32_t *op;  // N * T dwords
+  template <int K>
+  __device__ void dma(const void *src, int part) const {
+    if (K % NS == part)
+      __builtin_amdgcn_global_load_lds(
+          (__attribute__((address_space(1))) void *)(src),
+          (__attribute__((address_space(3))) void *)(op + K * T +
+                                                     __builtin_amdgcn_readfirstlane(threadIdx.x & (T - 64))),
+          4, 0, 0);
+  }
+  // dword K, dwords K and K + 1: a value's own address
+  template <int K>
+  __device__ void fetch(const float *src, int part) const { dma<K>(src, part); }
+  template <int K>
+  __device__ void fetch(const double *src, int part) const {
+    dma<K>(src, part);
+    dma<K + 1>(reinterpret_cast<const char *>(src) + 4, part);
+  }
+  // f(part) for the wavefront's part, a constant in each copy of f's code
+  template <class F>
+  __device__ static void share(F &&f) {
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / T);
+    unroll<0, NS>([&](auto P) {
+      if (part == decltype(P)::value) f(P);
+    });
+  }
+  __device__ float f32(int k) const { return __uint_as_float(op[k * T + threadIdx.x]); }
+  __device__ double f64(int k) const {
+    return __hiloint2double((int)op[(k + 1) * T + threadIdx.x], (int)op[k * T + threadIdx.x]);
+  }
+  template <class V>
+  __device__ V value(int k) const {
+    if constexpr (std::is_same<V, double>::value) return f64(k);
+    else return f32(k);
+  }
+};
+
 // ------------------------------------------------------------------ forward
-// The epilogue operands that do not depend on the product are loaded before
-// it, from addresses valid for every thread (threads without an output read
-// right-hand side 0), so no load is predicated and the product's loads are
-// issued without waiting for them: the X rows always, and, with 8 wavefronts
-// of FP32 or BF16 operands (16 wavefronts leave no registers for them, and
-// the FP64 operands take them), the right-hand side and coefficients of the
-// first march row and of the closure row.
-template <class KT, int W, int MBW, class FT>
-__global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_fwd_kernel(FusedFwdArgs p) {
-  __shared__ typename KT::Acc red[W * 256 * MBW];
-  constexpr bool PF = !std::is_same<KT, KF64>::value && W == 8;
-  span_begin(p.tspan);
-  int tile, mbg;
-  if (tile_of(blockIdx.x, p.ntiles, p.nmb, tile, mbg)) {
-    const int t = threadIdx.x;
-    const int col = t & 15;
-    const int m = 16 * MBW * mbg + (t >> 4);
-    const int steps = p.steps;
-    const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
+// Output t of a forward workgroup: right-hand side m (mm: 0 past the last) and
+// tile column col.
+struct FwdCol {
+  int col, m, mm, c, pc, xc, xcw, xce;
+  bool halo;
+  // T: outputs per workgroup (a thread past them reads right-hand side 0)
+  __device__ __forceinline__ FwdCol(const FusedFwdArgs &p, int tile, int mb0, int t, int T) {
+    const int i2 = p.i2, i0 = i2 + 2;
+    col = t & 15;
+    m = 16 * mb0 + (t >> 4);
+    mm = t < T && m < p.M ? m : 0;
     // interior column (1-based, before wrapping) of this lane's tile column
-    const int c = tile * (16 - 2 * steps) - steps + 1 + col;
-    int pc;
-    bool halo = false;
+    c = tile * (16 - 2 * p.steps) - p.steps + 1 + col;
+    halo = false;
     if (p.periodic) {
       pc = ((c - 1) % i2 + i2) % i2 + 1;
-    } else {
-      halo = c < 1 || c > i2;  // Dirichlet columns: X holds the boundary values
-      pc = min(max(c, 1), i2);
-    }
-    const int xc = halo ? (c < 1 ? 1 : i0) : pc + 1;  // X column
-    // X columns of the west and east neighbours (wrapped, or the Dirichlet
-    // column at the edge)
-    int xcw, xce;
-    if (p.periodic) {
+      // X columns of the west and east neighbours (wrapped, or the Dirichlet
+      // column at the edge)
       xcw = (pc == 1 ? i2 : pc - 1) + 1;
       xce = (pc == i2 ? 1 : pc + 1) + 1;
     } else {
+      halo = c < 1 || c > i2;  // Dirichlet columns: X holds the boundary values
+      pc = min(max(c, 1), i2);
       xcw = max(min(c - 1, i2 + 1), 0) + 1;
       xce = max(min(c + 1, i2 + 1), 0) + 1;
     }
-    const bool out = col >= steps && col < 16 - steps && c >= 1 && c <= i2;
-    const bool act = t < 256 * MBW && m < p.M;
-    const int mm = act ? m : 0;
-    double *x = p.x + (long)mm * p.x_stride;
-    const FT *f = rhs_ptr<FT>(p.f, p.f64) + (long)mm * p.f_stride;
+    xc = halo ? (c < 1 ? 1 : i0) : pc + 1;  // X column
+  }
+};
+
+// The epilogue operands that do not depend on the product are X(., JS),
+// X(., JS+1) with its west and east neighbours, X(., IE+1), and the coefficients
+// and right-hand side of the first march row and of the closure row.  They are
+// requested before it, from addresses valid for every thread (threads without
+// an output read right-hand side 0), so no load is predicated and the product's
+// loads are issued without waiting for them: all of them by DMA in FP64; the X
+// values into registers otherwise, and with 8 wavefronts the others too (16
+// wavefronts leave no registers for them).
+template <class KT, int W, int MBW, class FT>
+__global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_fwd_kernel(FusedFwdArgs p) {
+  constexpr int kVs = 0, kVc = 2, kFw = 4, kFe = 6, kNorth = 8, kRow1 = 10, kRowR = 15, kF1 = 20,
+                kFr = 20 + sizeof(FT) / 4, kN = 20 + sizeof(FT) / 2;
+  __shared__ typename KT::Acc red[W * 256 * MBW];
+  constexpr bool DM = std::is_same<KT, KF64>::value, PF = !DM && W == 8;
+  __shared__ uint32_t opmem[DM ? kN * 256 * MBW : 1];
+  const Operands<W, MBW, kN> ops{opmem};
+  span_begin(p.tspan);
+  int tile, mbg;
+  if (tile_of(blockIdx.x, p.ntiles, p.nmb, tile, mbg)) {
+    const int steps = p.steps;
+    const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
     const int js = p.js, jf = p.jf, ieb = p.ieb;
     const int jr = ieb - 1;                  // closure row
     const int j1 = steps > 0 ? js : jr;     // first march row (a valid row either way)
-    const long co = pc - 1;
-    auto cf = [&](const float *arr, int j) -> double { return (double)arr[co + (long)(j - 1) * i2]; };
-    auto fv = [&](int j) -> double { return (double)f[co + (long)(j - 1) * i2]; };
+    const int tid = DM ? threadIdx.x & (256 * MBW - 1) : threadIdx.x;
+    int pcol;
+    double vs, vc, fw, fe, xnorth;
+    FT f1, fr;
+    float c1[5], cr[5];
     // the free row's neighbours come from memory (that row is not written
     // in the forward pass), so the first row operation is exact in every
     // lane and each later one loses one lane per side
-    double vs = x[f2(i0, xc, js)];
-    double vc = x[f2(i0, xc, js + 1)];
-    const double fw = x[f2(i0, xcw, js + 1)];
-    const double fe = x[f2(i0, xce, js + 1)];
-    const double xnorth = x[f2(i0, xc, ieb + 1)];
-    FT f1 = 0, fr = 0;
-    float a1 = 0.f, b1 = 0.f, c1 = 0.f, d1 = 0.f, e1 = 0.f;
-    float ar = 0.f, br = 0.f, cr = 0.f, dr = 0.f, er = 0.f;
-    if constexpr (PF) {  // kept in their own precision until used
-      const long o1 = co + (long)(j1 - 1) * i2, orr = co + (long)(jr - 1) * i2;
-      f1 = f[o1];
-      a1 = p.ax[o1]; b1 = p.ay[o1]; c1 = p.bb[o1]; d1 = p.cx[o1]; e1 = p.cy[o1];
-      fr = f[orr];
-      ar = p.ax[orr]; br = p.ay[orr]; cr = p.bb[orr]; dr = p.cx[orr]; er = p.cy[orr];
+    {
+      const FwdCol o(p, tile, MBW * mbg, tid, 256 * MBW);
+      pcol = o.pc - 1;
+      const double *x = p.x + (long)o.mm * p.x_stride;
+      const FT *f = rhs_ptr<FT>(p.f, p.f64) + (long)o.mm * p.f_stride;
+      const long o1 = pcol + (long)(j1 - 1) * i2, orr = pcol + (long)(jr - 1) * i2;
+      const float *const cfs[5] = {p.ax, p.ay, p.bb, p.cx, p.cy};
+      if constexpr (DM) {
+        ops.share([&](auto part) {
+          ops.template fetch<kVs>(x + f2(i0, o.xc, js), part);
+          ops.template fetch<kVc>(x + f2(i0, o.xc, js + 1), part);
+          ops.template fetch<kFw>(x + f2(i0, o.xcw, js + 1), part);
+          ops.template fetch<kFe>(x + f2(i0, o.xce, js + 1), part);
+          ops.template fetch<kNorth>(x + f2(i0, o.xc, ieb + 1), part);
+          unroll<0, 5>([&](auto I) {
+            constexpr int i = decltype(I)::value;
+            ops.template fetch<kRow1 + i>(cfs[i] + o1, part);
+            ops.template fetch<kRowR + i>(cfs[i] + orr, part);
+          });
+          ops.template fetch<kF1>(f + o1, part);
+          ops.template fetch<kFr>(f + orr, part);
+        });
+      } else {
+        vs = x[f2(i0, o.xc, js)];
+        vc = x[f2(i0, o.xc, js + 1)];
+        fw = x[f2(i0, o.xcw, js + 1)];
+        fe = x[f2(i0, o.xce, js + 1)];
+        xnorth = x[f2(i0, o.xc, ieb + 1)];
+        if constexpr (PF) {  // kept in their own precision until used
+          f1 = f[o1];
+          fr = f[orr];
+#pragma unroll
+          for (int i = 0; i < 5; ++i) {
+            c1[i] = cfs[i][o1];
+            cr[i] = cfs[i][orr];
+          }
+        }
+      }
     }
     const double d = product_tile<KT, W, MBW>((const typename KT::A *)p.a, MBW * mbg, (p.M + 15) >> 4,
-                                              (const typename KT::B *)p.b, pc - 1, i2, red);
-    if (act) {
+                                              (const typename KT::B *)p.b, pcol, i2, red);
+    int again = tid;
+    if constexpr (DM) asm volatile("" : "+v"(again));  // worked out anew rather than kept in registers
+    const FwdCol o(p, tile, MBW * mbg, again, 256 * MBW);
+    const bool out = o.col >= steps && o.col < 16 - steps && o.c >= 1 && o.c <= i2;
+    if (threadIdx.x < 256 * MBW && o.m < p.M) {
+      const int m = o.m, pc = o.pc, xc = o.xc;
+      const bool halo = o.halo;
+      const long co = pc - 1;
+      double *x = p.x + (long)m * p.x_stride;
+      const FT *f = rhs_ptr<FT>(p.f, p.f64) + (long)m * p.f_stride;
+      auto cf = [&](const float *arr, int j) -> double { return (double)arr[co + (long)(j - 1) * i2]; };
+      auto fv = [&](int j) -> double { return (double)f[co + (long)(j - 1) * i2]; };
+      if constexpr (DM) {
+        vs = ops.f64(kVs);
+        vc = ops.f64(kVc);
+        fw = ops.f64(kFw);
+        fe = ops.f64(kFe);
+        xnorth = ops.f64(kNorth);
+        f1 = ops.template value<FT>(kF1);
+        fr = ops.template value<FT>(kFr);
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+          c1[i] = ops.f32(kRow1 + i);
+          cr[i] = ops.f32(kRowR + i);
+        }
+      } else if constexpr (!PF) {
+        const long o1 = co + (long)(j1 - 1) * i2, orr = co + (long)(jr - 1) * i2;
+        f1 = f[o1];
+        c1[0] = p.ax[o1]; c1[1] = p.ay[o1]; c1[2] = p.bb[o1]; c1[3] = p.cx[o1]; c1[4] = p.cy[o1];
+        fr = f[orr];
+        cr[0] = p.ax[orr]; cr[1] = p.ay[orr]; cr[2] = p.bb[orr]; cr[3] = p.cx[orr]; cr[4] = p.cy[orr];
+      }
       if (!halo) vs = vs - d;  // the south row as block b's correction leaves it
       if (p.d_out && out) p.d_out[(long)m * i2 + pc - 1] = d;
       for (int j = js; j <= jf; ++j) {
         const double sw = row_shr1(vc), se = row_shl1(vc);
         const double xw = j == js ? fw : sw, xe = j == js ? fe : se;
         double r;
-        if (PF && j == js)
-          r = ((double)f1 - (double)a1 * xw - (double)b1 * vs - (double)c1 * vc - (double)d1 * xe) /
-              (double)e1;
+        if (j == js)
+          r = ((double)f1 - (double)c1[0] * xw - (double)c1[1] * vs - (double)c1[2] * vc - (double)c1[3] * xe) /
+              (double)c1[4];
         else
           r = (fv(j) - cf(p.ax, j) * xw - cf(p.ay, j) * vs - cf(p.bb, j) * vc - cf(p.cx, j) * xe) /
               cf(p.cy, j);
@@ -326,13 +458,8 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
       }
       const double sw = row_shr1(vc), se = row_shl1(vc);
       const double xw = steps == 0 ? fw : sw, xe = steps == 0 ? fe : se;
-      double e;
-      if constexpr (PF)
-        e = (double)fr - (double)ar * xw - (double)br * vs - (double)cr * vc - (double)dr * xe -
-            (double)er * xnorth;
-      else
-        e = fv(jr) - cf(p.ax, jr) * xw - cf(p.ay, jr) * vs - cf(p.bb, jr) * vc - cf(p.cx, jr) * xe -
-            cf(p.cy, jr) * xnorth;
+      const double e = (double)fr - (double)cr[0] * xw - (double)cr[1] * vs - (double)cr[2] * vc -
+                       (double)cr[3] * xe - (double)cr[4] * xnorth;
       if (out) {
         const long eo = lt_index(m, (int)co, nchk);
         if (p.e_out) p.e_out[eo] = e;
@@ -347,15 +474,19 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
 // Workgroups [0, nhom_wg): the homogeneous march of block b+1, one wavefront
 // per (tile, RHS), first so that the launch's longest dependent chain starts
 // at once; then the product tiles of RINV_b (with the epilogue), then, when
-// W_b is given, those of W_b (the coupling row, only stored).  The
-// epilogue's X operands (and, where the forward kernel loads them early, its
-// right-hand side and coefficients) are loaded before the product from
-// clamped addresses (column I2 for lanes past it, row 1 for the closure row
-// of the first block, which has none).
+// W_b is given, those of W_b (the coupling row, only stored).  The epilogue
+// operands (five X values, the right-hand side and coefficients of the closure
+// row of block b-1 and the forward correction of its south row) are requested
+// where the forward kernel does, from clamped addresses (column I2 for lanes
+// past it, row 1 for the closure row of the first block, which has none).
 template <class KT, int W, int MBW, class FT>
 __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_bwd_kernel(FusedBwdArgs p) {
+  constexpr int kFree = 0, kSouth = 2, kCen = 4, kW = 6, kE = 8, kDs = 10, kRow = 12, kF = 17,
+                kN = 17 + sizeof(FT) / 4;
   __shared__ typename KT::Acc red[W * 256 * MBW];
-  constexpr bool PF = !std::is_same<KT, KF64>::value && W == 8;
+  constexpr bool DM = std::is_same<KT, KF64>::value, PF = !DM && W == 8;
+  __shared__ uint32_t opmem[DM ? kN * 256 * MBW : 1];
+  const Operands<W, MBW, kN> ops{opmem};
   span_begin(p.tspan);
   const int wg = blockIdx.x;
   int tile, mbg;
@@ -368,56 +499,88 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
     const int wp = wg - p.nhom_wg;
     const bool cpl = wp >= p.nprod_half;
     if (tile_of(cpl ? wp - p.nprod_half : wp, p.ntiles, p.nmb, tile, mbg)) {
-      const int t = threadIdx.x;
-      const int m = 16 * MBW * mbg + (t >> 4);
+      const int tid = DM ? threadIdx.x & (256 * MBW - 1) : threadIdx.x;
       const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
-      const int c = 16 * tile + 1 + (t & 15);
-      const bool ok = c <= i2;
-      const bool act = t < 256 * MBW && m < p.M && ok;
-      const int mm = act ? m : 0, cc = min(c, i2);
       const int js = p.js, jrow = max(js - 1, 1);
-      double *x = p.x + (long)mm * p.x_stride;
-      const bool resid = !cpl && p.do_resid && act;
-      const long co = (long)(cc - 1) + (long)(jrow - 1) * i2;  // coefficient row js-1
-      const int xcw = p.periodic ? (cc == 1 ? i2 : cc - 1) + 1 : cc;
-      const int xce = p.periodic ? (cc == i2 ? 1 : cc + 1) + 1 : cc + 2;
-      const double *dsp = p.dsouth ? p.dsouth : p.hfree_out;  // any valid (M, i2) array
-      const FT *fp = rhs_ptr<FT>(p.f, p.f64) + (long)mm * p.f_stride + co;
-      const double *dp = dsp + (long)mm * i2 + cc - 1;
+      double xfree, xsouth, xcen, xw, xe, ds;
+      FT fr;
+      float cr[5];
       // closure row js-1 of block b-1; row js = IE(b-1)
-      const double xfree = x[f2(i0, cc + 1, js + 1)];
-      double xsouth = x[f2(i0, cc + 1, jrow)];
-      const double xcen = x[f2(i0, cc + 1, js)];
-      const double xw = x[f2(i0, xcw, js)];
-      const double xe = x[f2(i0, xce, js)];
-      FT fr = 0;
-      float ar = 0.f, br = 0.f, cr = 0.f, dr = 0.f, er = 0.f;
-      double ds = 0.0;
-      if constexpr (PF) {
-        fr = *fp;
-        ar = p.ax[co]; br = p.ay[co]; cr = p.bb[co]; dr = p.cx[co]; er = p.cy[co];
-        ds = *dp;
+      const double *dsp = p.dsouth ? p.dsouth : p.hfree_out;  // any valid (M, i2) array
+      const float *const cfs[5] = {p.ax, p.ay, p.bb, p.cx, p.cy};
+      if (!DM || !cpl) {
+        const int m = 16 * MBW * mbg + (tid >> 4), mm = tid < 256 * MBW && m < p.M ? m : 0;
+        const int cc = min(16 * tile + 1 + (tid & 15), i2);
+        const double *x = p.x + (long)mm * p.x_stride;
+        const long co = (long)(cc - 1) + (long)(jrow - 1) * i2;  // coefficient row js-1
+        const int xcw = p.periodic ? (cc == 1 ? i2 : cc - 1) + 1 : cc;
+        const int xce = p.periodic ? (cc == i2 ? 1 : cc + 1) + 1 : cc + 2;
+        const FT *fp = rhs_ptr<FT>(p.f, p.f64) + (long)mm * p.f_stride + co;
+        const double *dp = dsp + (long)mm * i2 + cc - 1;
+        if constexpr (DM) {
+          ops.share([&](auto part) {
+            ops.template fetch<kFree>(x + f2(i0, cc + 1, js + 1), part);
+            ops.template fetch<kSouth>(x + f2(i0, cc + 1, jrow), part);
+            ops.template fetch<kCen>(x + f2(i0, cc + 1, js), part);
+            ops.template fetch<kW>(x + f2(i0, xcw, js), part);
+            ops.template fetch<kE>(x + f2(i0, xce, js), part);
+            ops.template fetch<kDs>(dp, part);
+            unroll<0, 5>([&](auto I) {
+              constexpr int i = decltype(I)::value;
+              ops.template fetch<kRow + i>(cfs[i] + co, part);
+            });
+            ops.template fetch<kF>(fp, part);
+          });
+        } else {
+          xfree = x[f2(i0, cc + 1, js + 1)];
+          xsouth = x[f2(i0, cc + 1, jrow)];
+          xcen = x[f2(i0, cc + 1, js)];
+          xw = x[f2(i0, xcw, js)];
+          xe = x[f2(i0, xce, js)];
+          if constexpr (PF) {
+            fr = *fp;
+            ds = *dp;
+#pragma unroll
+            for (int i = 0; i < 5; ++i) cr[i] = cfs[i][co];
+          }
+        }
       }
       // lanes past I2 (last tile) read the zero-padded matrix columns
       const double v = product_tile<KT, W, MBW>((const typename KT::A *)p.a, MBW * mbg, (p.M + 15) >> 4,
-                                                (const typename KT::B *)(cpl ? p.bw : p.b), c - 1, i2, red);
-      if (act) {
+                                                (const typename KT::B *)(cpl ? p.bw : p.b), 16 * tile + (tid & 15), i2,
+                                                red);
+      int again = tid;
+      if constexpr (DM) asm volatile("" : "+v"(again));  // as in the forward kernel
+      const int m = 16 * MBW * mbg + (again >> 4), c = 16 * tile + 1 + (again & 15);
+      if (threadIdx.x < 256 * MBW && m < p.M && c <= i2) {
         const long ro = (long)m * i2 + c - 1;
         if (cpl) {
           p.hcpl_out[ro] = v;
         } else {
           p.hfree_out[ro] = v;
+          if constexpr (DM) xfree = ops.f64(kFree);
           const double north = xfree + v;
-          x[f2(i0, c + 1, js + 1)] = north;
-          if (resid) {
-            if constexpr (!PF) {
-              fr = *fp;
-              ar = p.ax[co]; br = p.ay[co]; cr = p.bb[co]; dr = p.cx[co]; er = p.cy[co];
-              ds = *dp;
+          p.x[(long)m * p.x_stride + f2(i0, c + 1, js + 1)] = north;
+          if (p.do_resid) {
+            if constexpr (DM) {
+              xsouth = ops.f64(kSouth);
+              xcen = ops.f64(kCen);
+              xw = ops.f64(kW);
+              xe = ops.f64(kE);
+              ds = ops.f64(kDs);
+              fr = ops.template value<FT>(kF);
+#pragma unroll
+              for (int i = 0; i < 5; ++i) cr[i] = ops.f32(kRow + i);
+            } else if constexpr (!PF) {
+              const long co = (long)(c - 1) + (long)(jrow - 1) * i2;
+              fr = rhs_ptr<FT>(p.f, p.f64)[(long)m * p.f_stride + co];
+              ds = dsp[ro];
+#pragma unroll
+              for (int i = 0; i < 5; ++i) cr[i] = cfs[i][co];
             }
             if (p.dsouth) xsouth = xsouth - ds;
-            const double e = (double)fr - (double)ar * xw - (double)br * xsouth - (double)cr * xcen -
-                             (double)dr * xe - (double)er * north;
+            const double e = (double)fr - (double)cr[0] * xw - (double)cr[1] * xsouth - (double)cr[2] * xcen -
+                             (double)cr[3] * xe - (double)cr[4] * north;
             const long eo = lt_index(m, c - 1, nchk);
             if (p.e_out) p.e_out[eo] = e;
             if (p.e32_out) p.e32_out[eo] = (float)e;
