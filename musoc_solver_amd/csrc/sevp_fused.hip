@@ -29,6 +29,10 @@
 //     the next launch (its workgroups come first), when every column is
 //     complete.
 //
+// The last workgroups of a launch read the next launch's matrices into L2: a
+// launch is a chain of latencies (operands, product, epilogue) with the memory
+// idle for most of it.
+//
 // A pass is 2*NB0 + 1 launches instead of 4*NB0 + 2, each influence matrix is
 // read from HBM once for all right-hand sides, and no partial products go
 // through memory.  Both operands are in lane tiles, so a wavefront's operand
@@ -242,6 +246,32 @@ __device__ __forceinline__ bool tile_of(int wg, int ntiles, int nmb, int &tile, 
   return tile < ntiles;
 }
 
+// Workgroup wg of the last ones of a launch: the matrix columns that the next
+// launch's workgroups of one column tile read (n(i), i = 0..15), a line a lane,
+// into the L2 of their XCD.  The memory is idle for most of a launch, and the
+// next one begins with reading its matrix.
+template <class KT, int W, class F>
+__device__ __forceinline__ void warm_next(int wg, int ntiles, const void *next, int nchk, F &&n) {
+  constexpr int STEP = 128 / (int)sizeof(typename KT::BV);  // columns a line
+  constexpr int NS = STEP < 16 ? 16 / STEP + 1 : 2;         // lines that 16 columns may lie in, per q
+  constexpr int CPI = 64 / (4 * NS);                        // chunks an instruction
+  __shared__ uint32_t into[64];
+  int tile, mb;
+  if (!tile_of(wg, ntiles, 1, tile, mb)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int q = lane & 3, k = (lane >> 2) % NS, sub = lane / (4 * NS);
+  const int col = n(tile, min(k * STEP, 15));
+  const typename KT::B *src = static_cast<const typename KT::B *>(next) +
+                              ((long)(col >> 4) * nchk * 64 + (col & 15) + 16 * q) * 4;
+  for (int i = wave; i * CPI < nchk; i += W) {
+    const int ch = i * CPI + sub;
+    if (sub < CPI && ch < nchk)
+      __builtin_amdgcn_global_load_lds((__attribute__((address_space(1))) void *)(src + (long)ch * 256),
+                                       (__attribute__((address_space(3))) void *)(into), 4, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // The right-hand sides of a launch: FP32 (a solve's s) or FP64 (a
 // refinement residual), a template parameter so that their loads need no
 // branch.
@@ -352,7 +382,10 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
   const Operands<W, MBW, kN> ops{opmem};
   span_begin(p.tspan);
   int tile, mbg;
-  if (tile_of(blockIdx.x, p.ntiles, p.nmb, tile, mbg)) {
+  if (__builtin_expect((int)blockIdx.x >= p.nprod, 0)) {
+    warm_next<KT, W>(blockIdx.x - p.nprod, p.ntiles, p.next, (p.i2 + 15) >> 4,
+                     [&](int tl, int i) { return FwdCol(p, tl, 0, i, 16).pc - 1; });
+  } else if (tile_of(blockIdx.x, p.ntiles, p.nmb, tile, mbg)) {
     const int steps = p.steps;
     const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
     const int js = p.js, jf = p.jf, ieb = p.ieb;
@@ -496,9 +529,14 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
       march_body<1, MODE_HOM>(p.hom, (int)(wave % p.hom_tiles), (int)(wave / p.hom_tiles), 0, 1,
                               threadIdx.x & 63);
   } else {
-    const int wp = wg - p.nhom_wg;
+    const int wp = wg - p.nhom_wg, ww = wp - (p.bw ? 2 : 1) * p.nprod_half;
+    if (__builtin_expect(ww >= 0, 0)) {
+      const bool second = ww >= p.nwarm;
+      warm_next<KT, W>(second ? ww - p.nwarm : ww, p.ntiles, second ? p.nextw : p.next, (p.i2 + 15) >> 4,
+                       [](int tl, int i) { return 16 * tl + i; });
+    }
     const bool cpl = wp >= p.nprod_half;
-    if (tile_of(cpl ? wp - p.nprod_half : wp, p.ntiles, p.nmb, tile, mbg)) {
+    if (ww < 0 && tile_of(cpl ? wp - p.nprod_half : wp, p.ntiles, p.nmb, tile, mbg)) {
       const int tid = DM ? threadIdx.x & (256 * MBW - 1) : threadIdx.x;
       const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
       const int js = p.js, jrow = max(js - 1, 1);
@@ -610,10 +648,23 @@ static int rows_per_group(int arith, int M, int rows) {
   return arith != FUSED_F64 ? 2 : 1;
 }
 
-long fused_fwd_workgroups(const FusedFwdArgs &a) { return placed_workgroups(a.ntiles, a.nmb); }
+long fused_fwd_workgroups(const FusedFwdArgs &a) { return a.nprod + (a.next ? placed_workgroups(a.ntiles, 1) : 0); }
 
 long fused_bwd_workgroups(const FusedBwdArgs &a) {
-  return a.nhom_wg + (a.bw ? 2L : 1L) * a.nprod_half;
+  return a.nhom_wg + (a.bw ? 2L : 1L) * a.nprod_half + (a.next ? 1L : 0L) * a.nwarm + (a.nextw ? 1L : 0L) * a.nwarm;
+}
+
+// Whether a launch of wgs product workgroups brings the next one's matrices
+// near: while those (two going backward) are about what the L2s hold, 8 of 4 MiB,
+// or less, and the chip has room for the workgroups that do it beside the
+// product's.  Measured to 33 MB: refined solves, FP64 720 x 360 with one
+// right-hand side 3.15 -> 2.38 ms (2.89 by split K), 400 x 190 with one 1.31 ->
+// 1.10, 1040 x 500 with 8 5.85 -> 4.84 (5.25 by split K), 800 x 380 with 24 3.71 ->
+// 3.33; FP32 800 x 380 with one 7.50 -> 6.79, with 48 (336 workgroups going
+// backward) 10.0 -> 9.3, 1200 x 580 with 8 14.6 -> 13.1, with 40 (480) 20.3 -> 20.6.
+static bool warms(int arith, int i2, long wgs) {
+  const long n = (i2 + 15) / 16 * 16, elem = arith == FUSED_F64 ? 8 : (arith == FUSED_B16 ? 2 : 4);
+  return 2 * n * n * elem <= (36L << 20) && wgs <= 384;
 }
 
 static int waves_of(int w) { return w == 0 ? FUSED_WAVES : w; }
@@ -627,6 +678,8 @@ int fused_fwd_prepare(FusedFwdArgs &a, int arith) {
   a.ntiles = fused_tiles_fwd(a.i2, a.steps);
   a.mbw = rows_per_group(arith, a.M, a.rows);
   a.nmb = ((a.M + 15) / 16 + a.mbw - 1) / a.mbw;
+  a.nprod = (int)placed_workgroups(a.ntiles, a.nmb);
+  if (!warms(arith, a.i2, a.nprod)) a.next = nullptr;
   return 0;
 }
 
@@ -639,6 +692,8 @@ int fused_bwd_prepare(FusedBwdArgs &a, int arith) {
   a.mbw = rows_per_group(arith, a.M, a.rows);
   a.nmb = ((a.M + 15) / 16 + a.mbw - 1) / a.mbw;
   a.nprod_half = (int)placed_workgroups(a.ntiles, a.nmb);
+  a.nwarm = (int)placed_workgroups(a.ntiles, 1);
+  if (!warms(arith, a.i2, 2L * a.nprod_half)) a.next = a.nextw = nullptr;
   a.hom_tiles = 0;
   a.nhom_wg = 0;
   if (a.has_hom && a.hom.jf >= a.hom.js) {  // a one-row block has nothing to march

@@ -231,6 +231,7 @@ constexpr int FUSED_WAVES = 16;  // the default; 8 is the other compiled choice
 struct FusedFwdArgs {
   const void *a;      // e_b, lane tiles of (M, i2)
   const void *b;      // RINV1_b, lane tiles of (i2, i2)
+  const void *next;   // RINV1_(b+1), brought near for the next launch (may be null)
   int M, i2, periodic;
   // block b+1: march rows js .. jf (steps = jf - js + 1), closure row ieb - 1
   int js, jf, ieb, steps;
@@ -245,7 +246,9 @@ struct FusedFwdArgs {
   double *d_out;       // d itself (M, i2) row-major, kept when block b+1 is one row high (may be null)
   int waves;           // wavefronts per workgroup (8 or 16; 0: FUSED_WAVES)
   int rows;            // 16-row tiles per workgroup (1 or 2; 0: by arithmetic)
-  int ntiles, nmb, mbw;  // set by the launcher: column tiles, row-tile groups, row tiles per group
+  // set by the launcher: column tiles, row-tile groups, row tiles per group,
+  // product workgroups
+  int ntiles, nmb, mbw, nprod;
   unsigned long long *tspan;  // profiling: kernel span slot (null: off)
 };
 
@@ -256,6 +259,7 @@ struct FusedBwdArgs {
   const void *a;       // e_b, lane tiles
   const void *b;       // RINV_b, lane tiles
   const void *bw;      // W_b, lane tiles (null for the first block)
+  const void *next, *nextw;  // RINV_(b-1), W_(b-1), brought near for the next launch (may be null)
   int M, i2, periodic;
   int js;              // JS of block b (IE(b-1), or 1)
   int do_resid;        // b > 1: closure residual of block b-1 at row js-1
@@ -276,7 +280,7 @@ struct FusedBwdArgs {
   int has_hom;
   int waves;           // wavefronts per workgroup (8 or 16; 0: FUSED_WAVES)
   int rows;            // 16-row tiles per workgroup (1 or 2; 0: by arithmetic)
-  int ntiles, nmb, mbw, nprod_half, hom_tiles, nhom_wg;  // set by the launcher
+  int ntiles, nmb, mbw, nprod_half, nwarm, hom_tiles, nhom_wg;  // set by the launcher
   unsigned long long *tspan;
 };
 // Elements of the lane tiles of an (m, k) operand: 16-row by 16-column
