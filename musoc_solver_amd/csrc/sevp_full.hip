@@ -13,9 +13,9 @@
 // values, and a final pass (halo_fix_kernel) leaves the halo columns as the
 // reference leaves them.
 //
-// The correction products use a tiled FP64 GEMM whose every output is one
-// thread's sequential sum over k from zero with separately rounded multiply
-// and add: the reference's DUM2(N)=DUM2(N)+DUM1(M)*RINV(M,N) loop order.
+// The correction products keep every output one sequential sum over k from
+// zero with separately rounded multiply and add: the reference's
+// DUM2(N)=DUM2(N)+DUM1(M)*RINV(M,N) loop order.
 //
 // MATINV is the reference's Gauss-Jordan without pivoting
 // (PREP/template/GLOBAL/src/prep_GLOBAL.f90:516-568) with the matrix held in
