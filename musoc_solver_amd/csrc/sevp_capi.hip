@@ -645,7 +645,10 @@ static int run_fused_pass(const FullCtx &c, const float *f32, const double *f64,
     FusedFwdArgs a{};
     a.a = erow(b);
     a.b = opnd(c.rinv1_64t, c.rinv1_32, c.rinv1_16t, (b - 1) * tw);
-    if (c.fwarm && b + 1 < c.nb0) a.next = opnd(c.rinv1_64t, c.rinv1_32, c.rinv1_16t, b * tw);
+    if (c.fwarm && b + 1 < c.nb0) {
+      a.next = opnd(c.rinv1_64t, c.rinv1_32, c.rinv1_16t, b * tw);
+      a.next_steps = c.ie[b + 1] - c.ie[b] - 1;
+    }
     a.M = nrhs; a.i2 = c.i2; a.periodic = c.periodic;
     a.js = c.ie[b - 1]; a.jf = c.ie[b] - 2; a.ieb = c.ie[b];
     a.steps = a.jf - a.js + 1;

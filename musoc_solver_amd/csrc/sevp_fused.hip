@@ -48,6 +48,7 @@
 #include "sevp_dev.h"
 #include "sevp_internal.h"
 #include "sevp_march.h"
+#include "sevp_tiles.h"
 
 namespace sevp {
 
@@ -236,28 +237,18 @@ __device__ __forceinline__ double product_tile(const typename KT::A *alt, int mb
   return s;
 }
 
-// XCD-aware placement: workgroup id -> (column tile, 16-row block).  The
-// dispatcher deals workgroups to the 8 XCDs in turn; the row blocks of one
-// column tile get ids that land on the same XCD one after another.
-__device__ __forceinline__ bool tile_of(int wg, int ntiles, int nmb, int &tile, int &mb) {
-  const int xcd = wg & 7, slot = wg >> 3;
-  tile = (slot / nmb) * 8 + xcd;
-  mb = slot % nmb;
-  return tile < ntiles;
-}
-
 // Workgroup wg of the last ones of a launch: the matrix columns that the next
-// launch's workgroups of one column tile read (n(i), i = 0..15), a line a lane,
-// into the L2 of their XCD.  The memory is idle for most of a launch, and the
-// next one begins with reading its matrix.
+// launch's workgroups of one column tile read (n(tile, i), i = 0..15, of the
+// next launch's ntiles), a line a lane, into the L2 of their XCD.  The memory
+// is idle for most of a launch, and the next one begins with reading its matrix.
 template <class KT, int W, class F>
 __device__ __forceinline__ void warm_next(int wg, int ntiles, const void *next, int nchk, F &&n) {
   constexpr int STEP = 128 / (int)sizeof(typename KT::BV);  // columns a line
   constexpr int NS = STEP < 16 ? 16 / STEP + 1 : 2;         // lines that 16 columns may lie in, per q
   constexpr int CPI = 64 / (4 * NS);                        // chunks an instruction
   __shared__ uint32_t into[64];
-  int tile, mb;
-  if (!tile_of(wg, ntiles, 1, tile, mb)) return;
+  int tile;
+  if (!warm_tile(wg, ntiles, tile)) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int q = lane & 3, k = (lane >> 2) % NS, sub = lane / (4 * NS);
   const int col = n(tile, min(k * STEP, 15));
@@ -346,17 +337,16 @@ struct FwdCol {
     m = 16 * mb0 + (t >> 4);
     mm = t < T && m < p.M ? m : 0;
     // interior column (1-based, before wrapping) of this lane's tile column
-    c = tile * (16 - 2 * p.steps) - p.steps + 1 + col;
+    c = fused_fwd_column(tile, p.steps, col);
+    pc = fused_fwd_matrix_column(c, i2, p.periodic);
     halo = false;
     if (p.periodic) {
-      pc = ((c - 1) % i2 + i2) % i2 + 1;
       // X columns of the west and east neighbours (wrapped, or the Dirichlet
       // column at the edge)
       xcw = (pc == 1 ? i2 : pc - 1) + 1;
       xce = (pc == i2 ? 1 : pc + 1) + 1;
     } else {
       halo = c < 1 || c > i2;  // Dirichlet columns: X holds the boundary values
-      pc = min(max(c, 1), i2);
       xcw = max(min(c - 1, i2 + 1), 0) + 1;
       xce = max(min(c + 1, i2 + 1), 0) + 1;
     }
@@ -383,8 +373,9 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
   span_begin(p.tspan);
   int tile, mbg;
   if (__builtin_expect((int)blockIdx.x >= p.nprod, 0)) {
-    warm_next<KT, W>(blockIdx.x - p.nprod, p.ntiles, p.next, (p.i2 + 15) >> 4,
-                     [&](int tl, int i) { return FwdCol(p, tl, 0, i, 16).pc - 1; });
+    warm_next<KT, W>(blockIdx.x - p.nprod, p.next_tiles, p.next, (p.i2 + 15) >> 4, [&](int tl, int i) {
+      return fused_fwd_matrix_column(fused_fwd_column(tl, p.next_steps, i), p.i2, p.periodic) - 1;
+    });
   } else if (tile_of(blockIdx.x, p.ntiles, p.nmb, tile, mbg)) {
     const int steps = p.steps;
     const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
@@ -631,13 +622,6 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
 }
 
 // ---------------------------------------------------------------- launchers
-int fused_tiles_fwd(int i2, int steps) {
-  const int tout = 16 - 2 * steps;
-  return tout > 0 ? (i2 + tout - 1) / tout : 0;
-}
-
-static long placed_workgroups(int ntiles, int nmb) { return 8L * nmb * ((ntiles + 7) / 8); }
-
 // Row tiles per workgroup: the requested 1 or 2 (0: two for FP32 and BF16,
 // which share each matrix load, one for FP64), one when M <= 16.  Two row
 // tiles halve the matrix reads and the workgroups; FP64 then loads its
@@ -648,7 +632,9 @@ static int rows_per_group(int arith, int M, int rows) {
   return arith != FUSED_F64 ? 2 : 1;
 }
 
-long fused_fwd_workgroups(const FusedFwdArgs &a) { return a.nprod + (a.next ? placed_workgroups(a.ntiles, 1) : 0); }
+long fused_fwd_workgroups(const FusedFwdArgs &a) {
+  return a.nprod + (a.next ? placed_workgroups(a.next_tiles, 1) : 0);
+}
 
 long fused_bwd_workgroups(const FusedBwdArgs &a) {
   return a.nhom_wg + (a.bw ? 2L : 1L) * a.nprod_half + (a.next ? 1L : 0L) * a.nwarm + (a.nextw ? 1L : 0L) * a.nwarm;
@@ -679,6 +665,7 @@ int fused_fwd_prepare(FusedFwdArgs &a, int arith) {
   a.mbw = rows_per_group(arith, a.M, a.rows);
   a.nmb = ((a.M + 15) / 16 + a.mbw - 1) / a.mbw;
   a.nprod = (int)placed_workgroups(a.ntiles, a.nmb);
+  a.next_tiles = fused_tiles_fwd(a.i2, a.next_steps);
   if (!warms(arith, a.i2, a.nprod)) a.next = nullptr;
   return 0;
 }
@@ -701,7 +688,7 @@ int fused_bwd_prepare(FusedBwdArgs &a, int arith) {
     // same values; one keeps the march's registers within the product's)
     a.hom_tiles = march_tiles(a.hom, 1);
     if (a.hom_tiles <= 0) return -1;
-    a.nhom_wg = (int)(((long)a.hom_tiles * a.hom.nrhs + w - 1) / w);
+    a.nhom_wg = march_workgroups((long)a.hom_tiles * a.hom.nrhs, w);
   }
   return 0;
 }

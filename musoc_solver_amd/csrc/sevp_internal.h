@@ -232,6 +232,7 @@ struct FusedFwdArgs {
   const void *a;      // e_b, lane tiles of (M, i2)
   const void *b;      // RINV1_b, lane tiles of (i2, i2)
   const void *next;   // RINV1_(b+1), brought near for the next launch (may be null)
+  int next_steps;     // that launch's steps
   int M, i2, periodic;
   // block b+1: march rows js .. jf (steps = jf - js + 1), closure row ieb - 1
   int js, jf, ieb, steps;
@@ -247,8 +248,8 @@ struct FusedFwdArgs {
   int waves;           // wavefronts per workgroup (8 or 16; 0: FUSED_WAVES)
   int rows;            // 16-row tiles per workgroup (1 or 2; 0: by arithmetic)
   // set by the launcher: column tiles, row-tile groups, row tiles per group,
-  // product workgroups
-  int ntiles, nmb, mbw, nprod;
+  // product workgroups, the next launch's column tiles
+  int ntiles, nmb, mbw, nprod, next_tiles;
   unsigned long long *tspan;  // profiling: kernel span slot (null: off)
 };
 
@@ -288,7 +289,6 @@ struct FusedBwdArgs {
 __host__ __device__ inline long lane_tile_elems(int m, int k) {
   return (long)((m + 15) / 16) * ((k + 15) / 16) * 256;
 }
-int fused_tiles_fwd(int i2, int steps);
 // Set the launcher's fields (tiles, row blocks; K: the march lane width of
 // the backward launch's homogeneous march); nonzero if the shape is refused.
 int fused_fwd_prepare(FusedFwdArgs &a, int arith);
