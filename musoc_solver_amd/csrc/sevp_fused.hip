@@ -139,6 +139,12 @@ constexpr int min_waves_per_simd() {
   return two_per_cu<KT, W, MBW>() ? 8 : 1;
 }
 
+// Whether the epilogue's operands come by DMA (see Operands).
+template <class KT, int MBW>
+constexpr bool operands_by_dma() {
+  return std::is_same<KT, KF64>::value && MBW == 1;
+}
+
 // Partial tile of one wavefront over the chunks [c_lo, c_hi) of 16 k: MBW
 // 16-row tiles of A (row tiles mb0 .. mb0+MBW-1, clamped to the last one,
 // whose rows are then never stored) times the 16 columns of B around this
@@ -227,7 +233,7 @@ __device__ __forceinline__ double product_tile(const typename KT::A *alt, int mb
   for (int mb = 0; mb < MBW; ++mb)
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[(wave * MBW + mb) * 256 + KT::row(q, i) * 16 + (lane & 15)] = acc[mb][i];
-  if constexpr (std::is_same<KT, KF64>::value)
+  if constexpr (operands_by_dma<KT, MBW>())
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the epilogue's operands (Operands) too
   __syncthreads();
   double s = 0.0;
@@ -272,21 +278,24 @@ __device__ __forceinline__ const FT *rhs_ptr(const float *f, const double *f64) 
   else return f;
 }
 
-// FP64: the epilogue's operands that do not depend on the product, fetched
-// before it into LDS by DMA, so that they are on their way with the product's
-// operands, which take the registers, and there when the product is (720
-// columns, one right-hand side: 3.37 ms a solve with them loaded behind the
+// FP64, one row tile: the epilogue's operands that do not depend on the
+// product, fetched before it into LDS by DMA, so that they are on their way with
+// the product's operands, which take the registers, and there when the product is
+// (720 columns, one right-hand side: 3.37 ms a solve with them loaded behind the
 // product, 3.16 with these; 800 columns, 24: 3.83 and 3.71).  FP32 and BF16
 // launches are slower with these than with registers (8 wavefronts: 8.51 ms
 // against 8.35 at 800 columns) or without (16: 35.9 against 35.2 at 1440 x 720
-// with 64), their product's loads waiting behind them in every wavefront.
+// with 64), their product's loads waiting behind them in every wavefront; so are
+// FP64 launches of two row tiles, where the same wavefronts share twice the DMAs
+// out (a pass with 24 right-hand sides at 64 x 48, 8 wavefronts: 230 us against
+// 205; 16: 889 against 858 at 200 x 152, 3390 against 3270 at 720 x 360).
 //
 // Output t of the workgroup has dword k at op[k][t]; the wavefronts share the
-// dwords out (those of 256 MBW outputs each, every NS-th), all at the addresses
-// of output threadIdx.x % (256 MBW), so an address is valid for every thread.
-template <int W, int MBW, int N>
+// dwords out (those of 256 outputs each, every NS-th), all at the addresses
+// of output threadIdx.x % 256, so an address is valid for every thread.
+template <int W, int N>
 struct Operands {
-  static constexpr int T = 256 * MBW, NS = W / (4 * MBW);
+  static constexpr int T = 256, NS = W / 4;
   uint32_t *op;  // N * T dwords
   template <int K>
   __device__ void dma(const void *src, int part) const {
@@ -359,17 +368,18 @@ struct FwdCol {
 // and right-hand side of the first march row and of the closure row.  They are
 // requested before it, from addresses valid for every thread (threads without
 // an output read right-hand side 0), so no load is predicated and the product's
-// loads are issued without waiting for them: all of them by DMA in FP64; the X
-// values into registers otherwise, and with 8 wavefronts the others too (16
-// wavefronts leave no registers for them).
+// loads are issued without waiting for them: all of them by DMA in FP64 with one
+// row tile; the X values into registers otherwise, and with 8 wavefronts of FP32 or
+// BF16 the others too (16 wavefronts leave no registers for them, nor do the FP64
+// operands).
 template <class KT, int W, int MBW, class FT>
 __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_fwd_kernel(FusedFwdArgs p) {
   constexpr int kVs = 0, kVc = 2, kFw = 4, kFe = 6, kNorth = 8, kRow1 = 10, kRowR = 15, kF1 = 20,
                 kFr = 20 + sizeof(FT) / 4, kN = 20 + sizeof(FT) / 2;
   __shared__ typename KT::Acc red[W * 256 * MBW];
-  constexpr bool DM = std::is_same<KT, KF64>::value, PF = !DM && W == 8;
-  __shared__ uint32_t opmem[DM ? kN * 256 * MBW : 1];
-  const Operands<W, MBW, kN> ops{opmem};
+  constexpr bool DM = operands_by_dma<KT, MBW>(), PF = !std::is_same<KT, KF64>::value && W == 8;
+  __shared__ uint32_t opmem[DM ? kN * 256 : 1];
+  const Operands<W, kN> ops{opmem};
   span_begin(p.tspan);
   int tile, mbg;
   if (__builtin_expect((int)blockIdx.x >= p.nprod, 0)) {
@@ -382,7 +392,7 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
     const int js = p.js, jf = p.jf, ieb = p.ieb;
     const int jr = ieb - 1;                  // closure row
     const int j1 = steps > 0 ? js : jr;     // first march row (a valid row either way)
-    const int tid = DM ? threadIdx.x & (256 * MBW - 1) : threadIdx.x;
+    const int tid = DM ? threadIdx.x & 255 : threadIdx.x;
     int pcol;
     double vs, vc, fw, fe, xnorth;
     FT f1, fr;
@@ -508,9 +518,9 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
   constexpr int kFree = 0, kSouth = 2, kCen = 4, kW = 6, kE = 8, kDs = 10, kRow = 12, kF = 17,
                 kN = 17 + sizeof(FT) / 4;
   __shared__ typename KT::Acc red[W * 256 * MBW];
-  constexpr bool DM = std::is_same<KT, KF64>::value, PF = !DM && W == 8;
-  __shared__ uint32_t opmem[DM ? kN * 256 * MBW : 1];
-  const Operands<W, MBW, kN> ops{opmem};
+  constexpr bool DM = operands_by_dma<KT, MBW>(), PF = !std::is_same<KT, KF64>::value && W == 8;
+  __shared__ uint32_t opmem[DM ? kN * 256 : 1];
+  const Operands<W, kN> ops{opmem};
   span_begin(p.tspan);
   const int wg = blockIdx.x;
   int tile, mbg;
@@ -528,7 +538,7 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
     }
     const bool cpl = wp >= p.nprod_half;
     if (ww < 0 && tile_of(cpl ? wp - p.nprod_half : wp, p.ntiles, p.nmb, tile, mbg)) {
-      const int tid = DM ? threadIdx.x & (256 * MBW - 1) : threadIdx.x;
+      const int tid = DM ? threadIdx.x & 255 : threadIdx.x;
       const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
       const int js = p.js, jrow = max(js - 1, 1);
       double xfree, xsouth, xcen, xw, xe, ds;
