@@ -243,6 +243,24 @@ __device__ __forceinline__ double product_tile(const typename KT::A *alt, int mb
   return s;
 }
 
+// Kernel arguments in scalar registers from here on: loaded together, not one
+// part after another behind the branches that lead to their use (with
+// workgroup_id, a pass at 200 x 152, FP32, 8 wavefronts, one right-hand side: 663
+// us before, 637 with; 720 x 360 FP64, 16: 2250 and 2190).
+template <class T, class... More>
+__device__ __forceinline__ void have(T v, More... more) {
+  asm volatile("" ::"s"(v));
+  if constexpr (sizeof...(more) > 0) have(more...);
+}
+// blockIdx.x in a scalar register: what depends on it are then scalar
+// operations and branches.  (Behind span_begin's test of a lane the compiler
+// keeps it in a vector register, and masks each of a launch's parts by lanes.)
+__device__ __forceinline__ int workgroup_id() {
+  int wg = blockIdx.x;
+  asm volatile("" : "+s"(wg));
+  return wg;
+}
+
 // Workgroup wg of the last ones of a launch: the matrix columns that the next
 // launch's workgroups of one column tile read (n(tile, i), i = 0..15, of the
 // next launch's ntiles), a line a lane, into the L2 of their XCD.  The memory
@@ -380,13 +398,16 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
   constexpr bool DM = operands_by_dma<KT, MBW>(), PF = !std::is_same<KT, KF64>::value && W == 8;
   __shared__ uint32_t opmem[DM ? kN * 256 : 1];
   const Operands<W, kN> ops{opmem};
+  const int wg = workgroup_id();
+  have(p.ntiles, p.nmb, p.nprod, p.a, p.b, p.M, p.i2, p.periodic, p.js, p.jf, p.ieb, p.steps, p.x, p.x_stride);
+  have(p.ax, p.ay, p.bb, p.cx, p.cy, rhs_ptr<FT>(p.f, p.f64), p.f_stride);
   span_begin(p.tspan);
   int tile, mbg;
-  if (__builtin_expect((int)blockIdx.x >= p.nprod, 0)) {
-    warm_next<KT, W>(blockIdx.x - p.nprod, p.next_tiles, p.next, (p.i2 + 15) >> 4, [&](int tl, int i) {
+  if (__builtin_expect(wg >= p.nprod, 0)) {
+    warm_next<KT, W>(wg - p.nprod, p.next_tiles, p.next, (p.i2 + 15) >> 4, [&](int tl, int i) {
       return fused_fwd_matrix_column(fused_fwd_column(tl, p.next_steps, i), p.i2, p.periodic) - 1;
     });
-  } else if (tile_of(blockIdx.x, p.ntiles, p.nmb, tile, mbg)) {
+  } else if (tile_of(wg, p.ntiles, p.nmb, tile, mbg)) {
     const int steps = p.steps;
     const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
     const int js = p.js, jf = p.jf, ieb = p.ieb;
@@ -521,8 +542,10 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
   constexpr bool DM = operands_by_dma<KT, MBW>(), PF = !std::is_same<KT, KF64>::value && W == 8;
   __shared__ uint32_t opmem[DM ? kN * 256 : 1];
   const Operands<W, kN> ops{opmem};
+  const int wg = workgroup_id();
+  have(p.nhom_wg, p.ntiles, p.nmb, p.nprod_half, p.a, p.b, p.bw, p.M, p.i2, p.periodic, p.js, p.x, p.x_stride);
+  have(p.ax, p.ay, p.bb, p.cx, p.cy, rhs_ptr<FT>(p.f, p.f64), p.f_stride, p.dsouth, p.hfree_out);
   span_begin(p.tspan);
-  const int wg = blockIdx.x;
   int tile, mbg;
   if (wg < p.nhom_wg) {
     const long wave = (long)wg * W + (threadIdx.x >> 6);
