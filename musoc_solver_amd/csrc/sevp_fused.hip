@@ -145,13 +145,36 @@ constexpr bool operands_by_dma() {
   return std::is_same<KT, KF64>::value && MBW == 1;
 }
 
+// Chunks of 16 k per load group: 96 / W, one group at K <= 1536; half that for
+// FP64 with two row tiles and for the two-per-CU FP32 kernels.
+template <class KT, int W, int MBW>
+constexpr int load_group() {
+  return ((std::is_same<KT, KF64>::value && MBW == 2) || two_per_cu<KT, W, MBW>()) ? 48 / W : 96 / W;
+}
+// 1 / d of a group, rounded up.
+constexpr int share_of(int group, int d) { return (group + d - 1) / d; }
+
+// Whether there is a kernel in which a wavefront whose share is half or a
+// quarter of a group takes that: a load past the share is a repeated one, but a
+// compute unit takes 64 bytes a clock either way (one right-hand side, 720
+// columns, FP64: 3.52 ms a solve with twelve chunks for each wavefront's six,
+// 3.37 without; FP32, 8 wavefronts, 400 columns, 8: 3.26 and 2.77; 800, 24: 8.84
+// and 8.30).  Not where the registers are full with the whole group's: FP32 in 16
+// wavefronts.
+template <class KT, int W, int MBW>
+constexpr bool small_groups() {
+  return load_group<KT, W, MBW>() == 12 || (load_group<KT, W, MBW>() == 6 && MBW == 1) ||
+         std::is_same<KT, KF64>::value;
+}
+
 // Partial tile of one wavefront over the chunks [c_lo, c_hi) of 16 k: MBW
 // 16-row tiles of A (row tiles mb0 .. mb0+MBW-1, clamped to the last one,
 // whose rows are then never stored) times the 16 columns of B around this
 // lane's column n.  Chunks are loaded G at a time; a chunk past c_hi loads
 // the last one again and is skipped by the MFMA steps (the range is
-// wave-uniform), so no load is masked and none waits on another.
-template <class KT, int G, int MBW>
+// wave-uniform), so no load is masked and none waits on another.  PICK: a share
+// that half or a quarter of a group holds takes that.
+template <class KT, int G, bool PICK, int MBW>
 __device__ __forceinline__ void part_tile(const typename KT::A *alt, int mb0, int mtiles,
                                           const typename KT::B *blt, int n, int nchk, int c_lo,
                                           int c_hi, typename KT::CV (&acc)[MBW]) {
@@ -184,15 +207,9 @@ __device__ __forceinline__ void part_tile(const typename KT::A *alt, int mb0, in
 #pragma unroll
         for (int mb = 0; mb < MBW; ++mb) acc[mb] = KT::mma(av[g][mb], bv[g], acc[mb]);
   };
-  // A share that a smaller group holds takes that one: a load past the share
-  // is a repeated one, but a compute unit takes 64 bytes a clock either way (one
-  // right-hand side, 720 columns, FP64: 3.52 ms a solve with twelve chunks for
-  // each wavefront's six, 3.37 without; FP32, 8 wavefronts, 400 columns, 8: 3.26
-  // and 2.77; 800, 24: 8.84 and 8.30).  Not where the registers are full with
-  // the whole group's: FP32 in 16 wavefronts.
-  if constexpr (G == 12 || (G == 6 && MBW == 1) || std::is_same<KT, KF64>::value) {
-    typedef std::integral_constant<int, (G + 1) / 2> Half;
-    typedef std::integral_constant<int, (G + 3) / 4> Quarter;
+  if constexpr (PICK) {
+    typedef std::integral_constant<int, share_of(G, 2)> Half;
+    typedef std::integral_constant<int, share_of(G, 4)> Quarter;
     const int share = c_hi - c_lo;
     if (share <= Quarter::value) return group(Quarter{}, c_lo);
     if (share <= Half::value) return group(Half{}, c_lo);
@@ -210,12 +227,11 @@ __device__ __forceinline__ void part_tile(const typename KT::A *alt, int mb0, in
 }
 
 // The product tile of a workgroup: W wavefronts, each its share of the K
-// chunks (96 / W chunks per load group: one group at K <= 1536; half that
-// for FP64 with two row tiles and for the two-per-CU FP32 kernels); their
-// partial tiles go to LDS and thread t < 256 MBW receives the FP64 sum over
-// the wavefronts, in wavefront order, of row t / 16 (of the MBW row tiles)
-// and column t % 16 of the tile.  Every thread of the workgroup must call it.
-template <class KT, int W, int MBW>
+// chunks; their partial tiles go to LDS and thread t < 256 MBW receives the FP64
+// sum over the wavefronts, in wavefront order, of row t / 16 (of the MBW row
+// tiles) and column t % 16 of the tile.  Every thread of the workgroup must call
+// it.
+template <class KT, int W, int MBW, bool PICK>
 __device__ __forceinline__ double product_tile(const typename KT::A *alt, int mb0, int mtiles,
                                                const typename KT::B *blt, int n, int K,
                                                typename KT::Acc *red) {
@@ -226,9 +242,7 @@ __device__ __forceinline__ double product_tile(const typename KT::A *alt, int mb
   typename KT::CV acc[MBW];
 #pragma unroll
   for (int mb = 0; mb < MBW; ++mb) acc[mb] = typename KT::CV{0, 0, 0, 0};
-  constexpr int G =
-      ((std::is_same<KT, KF64>::value && MBW == 2) || two_per_cu<KT, W, MBW>()) ? 48 / W : 96 / W;
-  part_tile<KT, G, MBW>(alt, mb0, mtiles, blt, n, nchk, c_lo, c_hi, acc);
+  part_tile<KT, load_group<KT, W, MBW>(), PICK, MBW>(alt, mb0, mtiles, blt, n, nchk, c_lo, c_hi, acc);
 #pragma unroll
   for (int mb = 0; mb < MBW; ++mb)
 #pragma unroll
@@ -390,7 +404,7 @@ struct FwdCol {
 // row tile; the X values into registers otherwise, and with 8 wavefronts of FP32 or
 // BF16 the others too (16 wavefronts leave no registers for them, nor do the FP64
 // operands).
-template <class KT, int W, int MBW, class FT>
+template <class KT, int W, int MBW, bool PICK, class FT>
 __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_fwd_kernel(FusedFwdArgs p) {
   constexpr int kVs = 0, kVc = 2, kFw = 4, kFe = 6, kNorth = 8, kRow1 = 10, kRowR = 15, kF1 = 20,
                 kFr = 20 + sizeof(FT) / 4, kN = 20 + sizeof(FT) / 2;
@@ -460,7 +474,7 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
         }
       }
     }
-    const double d = product_tile<KT, W, MBW>((const typename KT::A *)p.a, MBW * mbg, (p.M + 15) >> 4,
+    const double d = product_tile<KT, W, MBW, PICK>((const typename KT::A *)p.a, MBW * mbg, (p.M + 15) >> 4,
                                               (const typename KT::B *)p.b, pcol, i2, red);
     int again = tid;
     if constexpr (DM) asm volatile("" : "+v"(again));  // worked out anew rather than kept in registers
@@ -534,7 +548,7 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
 // row of block b-1 and the forward correction of its south row) are requested
 // where the forward kernel does, from clamped addresses (column I2 for lanes
 // past it, row 1 for the closure row of the first block, which has none).
-template <class KT, int W, int MBW, class FT>
+template <class KT, int W, int MBW, bool PICK, class FT>
 __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_bwd_kernel(FusedBwdArgs p) {
   constexpr int kFree = 0, kSouth = 2, kCen = 4, kW = 6, kE = 8, kDs = 10, kRow = 12, kF = 17,
                 kN = 17 + sizeof(FT) / 4;
@@ -608,7 +622,7 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
         }
       }
       // lanes past I2 (last tile) read the zero-padded matrix columns
-      const double v = product_tile<KT, W, MBW>((const typename KT::A *)p.a, MBW * mbg, (p.M + 15) >> 4,
+      const double v = product_tile<KT, W, MBW, PICK>((const typename KT::A *)p.a, MBW * mbg, (p.M + 15) >> 4,
                                                 (const typename KT::B *)(cpl ? p.bw : p.b), 16 * tile + (tid & 15), i2,
                                                 red);
       int again = tid;
@@ -726,30 +740,48 @@ int fused_bwd_prepare(FusedBwdArgs &a, int arith) {
   return 0;
 }
 
-template <class KT, int W, int MBW, class FT>
+template <class KT, int W, int MBW, bool PICK, class FT>
 static void fwd_go(const FusedFwdArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
   const dim3 grid((unsigned)fused_fwd_workgroups(a)), block(64 * W);
-  if (ev0) hipExtLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, FT>), grid, block, 0, st, ev0, ev1, 0, a);
-  else hipLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, FT>), grid, block, 0, st, a);
+  if (ev0) hipExtLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, ev0, ev1, 0, a);
+  else hipLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, a);
 }
 
-template <class KT, int W, int MBW, class FT>
+template <class KT, int W, int MBW, bool PICK, class FT>
 static void bwd_go(const FusedBwdArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
   const dim3 grid((unsigned)fused_bwd_workgroups(a)), block(64 * W);
-  if (ev0) hipExtLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, FT>), grid, block, 0, st, ev0, ev1, 0, a);
-  else hipLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, FT>), grid, block, 0, st, a);
+  if (ev0) hipExtLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, ev0, ev1, 0, a);
+  else hipLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, a);
 }
 
 // the right-hand sides' precision -> the kernel that loads them
-template <class KT, int W, int MBW>
-static void go(const FusedFwdArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  if (a.f64) fwd_go<KT, W, MBW, double>(a, st, e0, e1);
-  else fwd_go<KT, W, MBW, float>(a, st, e0, e1);
+template <class KT, int W, int MBW, bool PICK>
+static void rhs_go(const FusedFwdArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  if (a.f64) fwd_go<KT, W, MBW, PICK, double>(a, st, e0, e1);
+  else fwd_go<KT, W, MBW, PICK, float>(a, st, e0, e1);
 }
-template <class KT, int W, int MBW>
-static void go(const FusedBwdArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  if (a.f64) bwd_go<KT, W, MBW, double>(a, st, e0, e1);
-  else bwd_go<KT, W, MBW, float>(a, st, e0, e1);
+template <class KT, int W, int MBW, bool PICK>
+static void rhs_go(const FusedBwdArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  if (a.f64) bwd_go<KT, W, MBW, PICK, double>(a, st, e0, e1);
+  else bwd_go<KT, W, MBW, PICK, float>(a, st, e0, e1);
+}
+
+// The kernel that picks load groups, where most wavefronts' shares are at most
+// half of one.  Elsewhere it costs: the choice takes registers and keeps the
+// operands requested ahead of the product from staying in flight over it (a pass
+// with 8 wavefronts: FP32 1440 x 120, 24 right-hand sides, one row tile 1347 us
+// with the choice, 1296 without; FP64 960 x 480, 48, two row tiles 6870, 6640;
+// BF16 1200 x 200, 48, one row tile 2260, 2000).  BF16 with few workgroups has
+// registers to spare and is faster with it at any width (1200 x 200, one
+// right-hand side: 1225, 1329).
+template <class KT, int W, int MBW, class Args>
+static void go(const Args &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  if constexpr (small_groups<KT, W, MBW>()) {
+    const int nchk = (a.i2 + 15) / 16, half = share_of(load_group<KT, W, MBW>(), 2);
+    if (2 * nchk <= (2 * half + 1) * W || (std::is_same<KT, KB16>::value && a.nmb == 1))
+      return rhs_go<KT, W, MBW, true>(a, st, e0, e1);
+  }
+  rhs_go<KT, W, MBW, false>(a, st, e0, e1);
 }
 
 // (arithmetic, waves, row tiles per workgroup) -> the compiled kernel
