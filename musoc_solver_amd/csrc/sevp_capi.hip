@@ -599,6 +599,8 @@ static int run_fused_pass(const FullCtx &c, const float *f32, const double *f64,
     if (c.farith == FUSED_B16) return b16t + off;
     return f32t + off;
   };
+  // RINV of every block, RINV1 and W of all but one
+  const long set = (3L * c.nb0 - 2) * tw * (c.farith == FUSED_F64 ? 8 : (c.farith == FUSED_B16 ? 2 : 4));
   double *E[2] = {c.fe, c.fe + c.fe_half};
   float *E32[2] = {c.fe32, c.fe32 + c.fe_half};
   double *HF[2] = {c.fh, c.fh + c.fhalf}, *HC[2] = {c.fhc, c.fhc + c.fhalf};
@@ -645,6 +647,7 @@ static int run_fused_pass(const FullCtx &c, const float *f32, const double *f64,
     FusedFwdArgs a{};
     a.a = erow(b);
     a.b = opnd(c.rinv1_64t, c.rinv1_32, c.rinv1_16t, (b - 1) * tw);
+    a.set = set;
     if (c.fwarm && b + 1 < c.nb0) {
       a.next = opnd(c.rinv1_64t, c.rinv1_32, c.rinv1_16t, b * tw);
       a.next_steps = c.ie[b + 1] - c.ie[b] - 1;
@@ -669,6 +672,7 @@ static int run_fused_pass(const FullCtx &c, const float *f32, const double *f64,
     FusedBwdArgs a{};
     a.a = erow(b);
     a.b = opnd(c.rinv64t, c.rinv32, c.rinv16t, (b - 1) * tw);
+    a.set = set;
     a.bw = (b == 1) ? nullptr : opnd(c.w64t, c.w32, c.w16t, (b - 2) * tw);
     if (c.fwarm && b > 1) a.next = opnd(c.rinv64t, c.rinv32, c.rinv16t, (b - 2) * tw);
     if (c.fwarm && b > 2) a.nextw = opnd(c.w64t, c.w32, c.w16t, (b - 3) * tw);

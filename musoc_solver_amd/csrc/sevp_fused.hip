@@ -404,7 +404,7 @@ struct FwdCol {
 // row tile; the X values into registers otherwise, and with 8 wavefronts of FP32 or
 // BF16 the others too (16 wavefronts leave no registers for them, nor do the FP64
 // operands).
-template <class KT, int W, int MBW, bool PICK, class FT>
+template <class KT, int W, int MBW, bool PICK, bool WARM, class FT>
 __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_fwd_kernel(FusedFwdArgs p) {
   constexpr int kVs = 0, kVc = 2, kFw = 4, kFe = 6, kNorth = 8, kRow1 = 10, kRowR = 15, kF1 = 20,
                 kFr = 20 + sizeof(FT) / 4, kN = 20 + sizeof(FT) / 2;
@@ -417,7 +417,7 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
   have(p.ax, p.ay, p.bb, p.cx, p.cy, rhs_ptr<FT>(p.f, p.f64), p.f_stride);
   span_begin(p.tspan);
   int tile, mbg;
-  if (__builtin_expect(wg >= p.nprod, 0)) {
+  if (WARM && __builtin_expect(wg >= p.nprod, 0)) {
     warm_next<KT, W>(wg - p.nprod, p.next_tiles, p.next, (p.i2 + 15) >> 4, [&](int tl, int i) {
       return fused_fwd_matrix_column(fused_fwd_column(tl, p.next_steps, i), p.i2, p.periodic) - 1;
     });
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
 // row of block b-1 and the forward correction of its south row) are requested
 // where the forward kernel does, from clamped addresses (column I2 for lanes
 // past it, row 1 for the closure row of the first block, which has none).
-template <class KT, int W, int MBW, bool PICK, class FT>
+template <class KT, int W, int MBW, bool PICK, bool WARM, class FT>
 __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fused_bwd_kernel(FusedBwdArgs p) {
   constexpr int kFree = 0, kSouth = 2, kCen = 4, kW = 6, kE = 8, kDs = 10, kRow = 12, kF = 17,
                 kN = 17 + sizeof(FT) / 4;
@@ -568,13 +568,13 @@ __global__ __launch_bounds__(64 * W, (min_waves_per_simd<KT, W, MBW>())) void fu
                               threadIdx.x & 63);
   } else {
     const int wp = wg - p.nhom_wg, ww = wp - (p.bw ? 2 : 1) * p.nprod_half;
-    if (__builtin_expect(ww >= 0, 0)) {
+    if (WARM && __builtin_expect(ww >= 0, 0)) {
       const bool second = ww >= p.nwarm;
       warm_next<KT, W>(second ? ww - p.nwarm : ww, p.ntiles, second ? p.nextw : p.next, (p.i2 + 15) >> 4,
                        [](int tl, int i) { return 16 * tl + i; });
     }
     const bool cpl = wp >= p.nprod_half;
-    if (ww < 0 && tile_of(cpl ? wp - p.nprod_half : wp, p.ntiles, p.nmb, tile, mbg)) {
+    if ((!WARM || ww < 0) && tile_of(cpl ? wp - p.nprod_half : wp, p.ntiles, p.nmb, tile, mbg)) {
       const int tid = DM ? threadIdx.x & 255 : threadIdx.x;
       const int i2 = p.i2, i0 = i2 + 2, nchk = (i2 + 15) >> 4;
       const int js = p.js, jrow = max(js - 1, 1);
@@ -695,9 +695,19 @@ long fused_bwd_workgroups(const FusedBwdArgs &a) {
 // 1.10, 1040 x 500 with 8 5.85 -> 4.84 (5.25 by split K), 800 x 380 with 24 3.71 ->
 // 3.33; FP32 800 x 380 with one 7.50 -> 6.79, with 48 (336 workgroups going
 // backward) 10.0 -> 9.3, 1200 x 580 with 8 14.6 -> 13.1, with 40 (480) 20.3 -> 20.6.
-static bool warms(int arith, int i2, long wgs) {
+//
+// Where all of a pass's matrices (`set` bytes) stay in the 256 MB last-level
+// cache from one pass to the next, they are near enough for wide launches, whose
+// workgroups leave no room for more (a pass with and without: FP32 1200 x 24, 196
+// MB, 8 right-hand sides 165 and 158 us; 1440 x 28, 232 MB, one 165 and 145; FP64
+// 960 x 24, 184 MB, 8 163 and 153; but FP64 1040 x 24, 294 MB, 8 224 and 251, 960 x
+// 40, 428 MB, 8 352 and 416).  Narrow ones still gain (FP64 720 x 24, 141 MB, 8 149
+// and 154), if they have a kernel to spare for it (warm_go).
+static bool warms(int arith, int i2, int waves, int mbw, long set, long wgs) {
   const long n = (i2 + 15) / 16 * 16, elem = arith == FUSED_F64 ? 8 : (arith == FUSED_B16 ? 2 : 4);
-  return 2 * n * n * elem <= (36L << 20) && wgs <= 384;
+  if (2 * n * n * elem > (36L << 20) || wgs > 384) return false;
+  if (set > 245000000L) return true;
+  return i2 <= 800 && (mbw == 1 || (arith != FUSED_F64 && waves == 8));
 }
 
 static int waves_of(int w) { return w == 0 ? FUSED_WAVES : w; }
@@ -713,7 +723,7 @@ int fused_fwd_prepare(FusedFwdArgs &a, int arith) {
   a.nmb = ((a.M + 15) / 16 + a.mbw - 1) / a.mbw;
   a.nprod = (int)placed_workgroups(a.ntiles, a.nmb);
   a.next_tiles = fused_tiles_fwd(a.i2, a.next_steps);
-  if (!warms(arith, a.i2, a.nprod)) a.next = nullptr;
+  if (!warms(arith, a.i2, w, a.mbw, a.set, a.nprod)) a.next = nullptr;
   return 0;
 }
 
@@ -727,7 +737,7 @@ int fused_bwd_prepare(FusedBwdArgs &a, int arith) {
   a.nmb = ((a.M + 15) / 16 + a.mbw - 1) / a.mbw;
   a.nprod_half = (int)placed_workgroups(a.ntiles, a.nmb);
   a.nwarm = (int)placed_workgroups(a.ntiles, 1);
-  if (!warms(arith, a.i2, 2L * a.nprod_half)) a.next = a.nextw = nullptr;
+  if (!warms(arith, a.i2, w, a.mbw, a.set, 2L * a.nprod_half)) a.next = a.nextw = nullptr;
   a.hom_tiles = 0;
   a.nhom_wg = 0;
   if (a.has_hom && a.hom.jf >= a.hom.js) {  // a one-row block has nothing to march
@@ -740,30 +750,42 @@ int fused_bwd_prepare(FusedBwdArgs &a, int arith) {
   return 0;
 }
 
-template <class KT, int W, int MBW, bool PICK, class FT>
+template <class KT, int W, int MBW, bool PICK, bool WARM, class FT>
 static void fwd_go(const FusedFwdArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
   const dim3 grid((unsigned)fused_fwd_workgroups(a)), block(64 * W);
-  if (ev0) hipExtLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, ev0, ev1, 0, a);
-  else hipLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, a);
+  if (ev0) hipExtLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, PICK, WARM, FT>), grid, block, 0, st, ev0, ev1, 0, a);
+  else hipLaunchKernelGGL((fused_fwd_kernel<KT, W, MBW, PICK, WARM, FT>), grid, block, 0, st, a);
 }
 
-template <class KT, int W, int MBW, bool PICK, class FT>
+template <class KT, int W, int MBW, bool PICK, bool WARM, class FT>
 static void bwd_go(const FusedBwdArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
   const dim3 grid((unsigned)fused_bwd_workgroups(a)), block(64 * W);
-  if (ev0) hipExtLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, ev0, ev1, 0, a);
-  else hipLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, PICK, FT>), grid, block, 0, st, a);
+  if (ev0) hipExtLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, PICK, WARM, FT>), grid, block, 0, st, ev0, ev1, 0, a);
+  else hipLaunchKernelGGL((fused_bwd_kernel<KT, W, MBW, PICK, WARM, FT>), grid, block, 0, st, a);
 }
 
 // the right-hand sides' precision -> the kernel that loads them
-template <class KT, int W, int MBW, bool PICK>
+template <class KT, int W, int MBW, bool PICK, bool WARM>
 static void rhs_go(const FusedFwdArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  if (a.f64) fwd_go<KT, W, MBW, PICK, double>(a, st, e0, e1);
-  else fwd_go<KT, W, MBW, PICK, float>(a, st, e0, e1);
+  if (a.f64) fwd_go<KT, W, MBW, PICK, WARM, double>(a, st, e0, e1);
+  else fwd_go<KT, W, MBW, PICK, WARM, float>(a, st, e0, e1);
 }
-template <class KT, int W, int MBW, bool PICK>
+template <class KT, int W, int MBW, bool PICK, bool WARM>
 static void rhs_go(const FusedBwdArgs &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  if (a.f64) bwd_go<KT, W, MBW, PICK, double>(a, st, e0, e1);
-  else bwd_go<KT, W, MBW, PICK, float>(a, st, e0, e1);
+  if (a.f64) bwd_go<KT, W, MBW, PICK, WARM, double>(a, st, e0, e1);
+  else bwd_go<KT, W, MBW, PICK, WARM, float>(a, st, e0, e1);
+}
+
+// The kernel without the part that brings the next matrices near, for launches
+// of two row tiles that do not: that part's code alone costs them (a pass with 24
+// right-hand sides, 16 wavefronts: FP32 64 x 48 271 us without it, 282 with, 200 x
+// 152 929, 977; FP64 800 x 24 224, 234).  The other kernels take as long either way, or are
+// faster with it (FP32, 8 wavefronts, 720 x 40: 1.02 of the time without).
+template <class KT, int W, int MBW, bool PICK, class Args>
+static void warm_go(const Args &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
+  if constexpr (MBW == 2 && (W == 16 || std::is_same<KT, KF64>::value))
+    if (!a.next) return rhs_go<KT, W, MBW, PICK, false>(a, st, e0, e1);
+  rhs_go<KT, W, MBW, PICK, true>(a, st, e0, e1);
 }
 
 // The kernel that picks load groups, where most wavefronts' shares are at most
@@ -779,9 +801,9 @@ static void go(const Args &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
   if constexpr (small_groups<KT, W, MBW>()) {
     const int nchk = (a.i2 + 15) / 16, half = share_of(load_group<KT, W, MBW>(), 2);
     if (2 * nchk <= (2 * half + 1) * W || (std::is_same<KT, KB16>::value && a.nmb == 1))
-      return rhs_go<KT, W, MBW, true>(a, st, e0, e1);
+      return warm_go<KT, W, MBW, true>(a, st, e0, e1);
   }
-  rhs_go<KT, W, MBW, false>(a, st, e0, e1);
+  warm_go<KT, W, MBW, false>(a, st, e0, e1);
 }
 
 // (arithmetic, waves, row tiles per workgroup) -> the compiled kernel

@@ -233,6 +233,7 @@ struct FusedFwdArgs {
   const void *b;      // RINV1_b, lane tiles of (i2, i2)
   const void *next;   // RINV1_(b+1), brought near for the next launch (may be null)
   int next_steps;     // that launch's steps
+  long set;           // bytes of all the matrices of a pass
   int M, i2, periodic;
   // block b+1: march rows js .. jf (steps = jf - js + 1), closure row ieb - 1
   int js, jf, ieb, steps;
@@ -261,6 +262,7 @@ struct FusedBwdArgs {
   const void *b;       // RINV_b, lane tiles
   const void *bw;      // W_b, lane tiles (null for the first block)
   const void *next, *nextw;  // RINV_(b-1), W_(b-1), brought near for the next launch (may be null)
+  long set;            // bytes of all the matrices of a pass
   int M, i2, periodic;
   int js;              // JS of block b (IE(b-1), or 1)
   int do_resid;        // b > 1: closure residual of block b-1 at row js-1
