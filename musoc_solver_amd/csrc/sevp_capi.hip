@@ -358,16 +358,8 @@ static int run_pre(const PreCtx &c, hipStream_t st) {
     HIPC(launch_matinv(c.rinv + (long)(nb - 1) * ww, sstride, c.w, c.nmat, c.zp, c.b1s, st));
     if (nb == c.nb0) break;
     for (int s = 0; s < c.nmat; ++s) {
-      GemmArgs gm{};
-      gm.a = c.rinv + s * sstride + (long)(nb - 1) * ww;
-      gm.a_sm = 1; gm.a_sk = c.w;
-      gm.b = c.rinv + s * sstride + (long)(c.nb0 - 1) * ww;
-      gm.b_sk = 1; gm.b_sn = c.w;
-      gm.M = c.w; gm.N = c.w; gm.K = c.w;
-      gm.ep = EP_NEGSUB;
-      gm.out = c.rinv1 + s * s1stride + (long)(nb - 1) * ww;
-      gm.out_ld = c.w;
-      HIPC(launch_gemm(gm, st));
+      HIPC(launch_square_product(c.rinv + s * sstride + (long)(nb - 1) * ww, c.rinv + s * sstride + (long)(c.nb0 - 1) * ww,
+                                 c.rinv1 + s * s1stride + (long)(nb - 1) * ww, c.w, true, st));
     }
     jl = jh;
   }
@@ -729,8 +721,8 @@ static int run_full_pass(const FullCtx &c, const float *f32, const double *f64, 
   auto corr = [&](const double *a, const double *b64, int ep, int xrow, double *dum0, double *out,
                   double *g, int cyrow) -> int {
     GemmArgs gm{};
-    gm.a = a; gm.a_sm = c.i2; gm.a_sk = 1;
-    gm.b = b64; gm.b_sk = 1; gm.b_sn = c.i2;
+    gm.a = a; gm.a_sm = c.i2;
+    gm.b = b64; gm.b_sn = c.i2;
     gm.M = nrhs; gm.N = c.i2; gm.K = c.i2;
     gm.ep = ep;
     gm.x = x; gm.x_stride = x_stride; gm.xrow = xrow;
@@ -1312,29 +1304,14 @@ static int build_products(sevp_plan p, const double *h_rinv, const double *h_rin
       m.rinv1_prev = (nb != 1) ? r1prev : nullptr;
       HIPC(launch_march(MODE_PRE, m, i2, st));
       HIPC(launch_matinv(cur.p, ww, i2, 1, p->zp.p, p->b1s.p, st));
-      if (nb != nb0) {
-        GemmArgs gm{};
-        gm.a = cur.p; gm.a_sm = 1; gm.a_sk = i2;
-        gm.b = tm.p; gm.b_sk = 1; gm.b_sn = i2;
-        gm.M = i2; gm.N = i2; gm.K = i2;
-        gm.ep = EP_NEGSUB;
-        gm.out = r1cur;
-        gm.out_ld = i2;
-        HIPC(launch_gemm(gm, st));
-      }
+      if (nb != nb0) HIPC(launch_square_product(cur.p, tm.p, r1cur, i2, true, st));
     }
     HIPC(launch_cvt_lane_tiles(cur.p, p->rinv32.p + (long)(nb - 1) * tw, i2, i2, 1, st));
     if (nb != nb0)
       HIPC(launch_cvt_lane_tiles(r1cur, p->rinv1_32.p + (long)(nb - 1) * tw, i2, i2, 1, st));
     if (nb >= 2) {  // W_nb = RINV_nb diag(CY(:, IE(nb-1)-1)) RINV1_(nb-1)
       HIPC(launch_scale_cols(cur.p, p->at(), jl - 1, i2, sc.p, st));
-      GemmArgs gm{};
-      gm.a = sc.p; gm.a_sm = 1; gm.a_sk = i2;
-      gm.b = r1prev; gm.b_sk = 1; gm.b_sn = i2;
-      gm.M = i2; gm.N = i2; gm.K = i2;
-      gm.ep = EP_COLMAJ;
-      gm.out = wt.p; gm.out_ld = i2;
-      HIPC(launch_gemm(gm, st));
+      HIPC(launch_square_product(sc.p, r1prev, wt.p, i2, false, st));
       HIPC(launch_cvt_lane_tiles(wt.p, p->w32.p + (long)(nb - 2) * tw, i2, i2, 1, st));
     }
     jl = jh;
@@ -1385,14 +1362,7 @@ static int make_low_precision_copies(sevp_plan p) {
     for (int nb = 2; nb <= p->d.nb0; ++nb) {
       const int js = p->ie[nb - 2];
       HIPC(launch_scale_cols(p->rinv.p + (long)(nb - 1) * ww, p->at(), js - 1, i2, t.p, p->stream));
-      GemmArgs gm{};
-      gm.a = t.p; gm.a_sm = 1; gm.a_sk = i2;
-      gm.b = p->rinv1.p + (long)(nb - 2) * ww; gm.b_sk = 1; gm.b_sn = i2;
-      gm.M = i2; gm.N = i2; gm.K = i2;
-      gm.ep = EP_COLMAJ;
-      gm.out = w.p;
-      gm.out_ld = i2;
-      HIPC(launch_gemm(gm, p->stream));
+      HIPC(launch_square_product(t.p, p->rinv1.p + (long)(nb - 2) * ww, w.p, i2, false, p->stream));
       const long off = (long)(nb - 2) * tw;
       if (b16) HIPC(launch_cvt_lane_tiles_bf16(w.p, p->w16t.p + off, i2, i2, 1, p->stream));
       else if (dbl) HIPC(launch_cvt_lane_tiles64(w.p, p->w64t.p + off, i2, i2, 1, p->stream));

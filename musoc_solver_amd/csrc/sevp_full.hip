@@ -27,6 +27,7 @@
 #include "sevp_dev.h"
 #include "sevp_internal.h"
 #include "sevp_march.h"
+#include "sevp_tiles.h"
 
 namespace sevp {
 
@@ -636,68 +637,54 @@ __global__ __launch_bounds__(192) void gemm_seq_few_kernel(GemmArgs p) {
   span_end(p.tspan);
 }
 
-// Square products of the influence build, D = A B (EP_COLMAJ) or
-// 0 - A B by successive subtractions (EP_NEGSUB): A and D with consecutive m
-// adjacent, B with consecutive k adjacent.  One output per thread, tile
-// 16 (m) x 16 (n), K in chunks of 64 staged through LDS.
+// Square products of the influence build, D = A B, or 0 - A B by successive
+// subtractions (neg): n x n column-major matrices, so A and D have consecutive m
+// adjacent and B consecutive k.  One output per thread, tile 16 (m) x 16 (n), K in
+// chunks of 64 staged through LDS.
 constexpr int GT_M = 16, GT_N = 16, GT_K = 64;
 
-__global__ __launch_bounds__(256) void gemm_square_kernel(GemmArgs p) {
+__global__ __launch_bounds__(256) void gemm_square_kernel(const double *a, const double *b, double *out,
+                                                          int n, int neg) {
   // both tiles k-contiguous (rows of GT_K + 2 doubles, 16-byte aligned) so a
   // thread reads two consecutive k of each operand with one 128-bit load
   __shared__ __align__(16) double As[GT_M][GT_K + 2];
   __shared__ __align__(16) double Bs[GT_N][GT_K + 2];
   const int t = threadIdx.x;
-  // XCD-aware placement: the dispatcher deals workgroups to the 8 XCDs in
-  // turn, so the row tiles of one column tile get ids on the same XCD, one
-  // after another, and read that tile of B from HBM once (the others from
-  // the XCD's L2); ids past the last column tile have no tile
-  const int ntn = (p.N + GT_N - 1) / GT_N, nmb = (p.M + GT_M - 1) / GT_M;
-  const int slot = blockIdx.x >> 3, tcol = (slot / nmb) * 8 + (blockIdx.x & 7);
-  if (tcol >= ntn) {
-    return;
-  }
-  const int n0 = tcol * GT_N, m0 = (slot % nmb) * GT_M;
+  // XCD-aware placement: the row tiles of one column tile read that tile of B
+  // from HBM once (the others from the XCD's L2); ids past the last column tile
+  // have no tile
+  const int ntl = (n + GT_N - 1) / GT_N;
+  int tcol, trow;
+  if (!tile_of(blockIdx.x, ntl, ntl, tcol, trow)) return;
+  const int n0 = tcol * GT_N, m0 = trow * GT_M;
   const int tn = t % GT_N, tm = t / GT_N;
-  // staging: each thread moves 4 elements of A and 4 of B per chunk
+  // staging: each thread moves 4 elements of A (m fastest) and 4 of B (k
+  // fastest) per chunk
   double ra[4], rb[4];
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int idx = t + 256 * q;
-      {  // A tile: kk fastest (contiguous when a_sk == 1)
-        const int kk = (p.a_sk == 1) ? idx % GT_K : idx / GT_M;
-        const int mm = (p.a_sk == 1) ? idx / GT_K : idx % GT_M;
-        const int m = m0 + mm, k = k0 + kk;
-        ra[q] = (m < p.M && k < p.K) ? p.a[(long)m * p.a_sm + (long)k * p.a_sk] : 0.0;
-      }
-      {  // B tile: kk fastest when b_sk == 1
-        const int kk = (p.b_sk == 1) ? idx % GT_K : idx / GT_N;
-        const int nn = (p.b_sk == 1) ? idx / GT_K : idx % GT_N;
-        const int n = n0 + nn, k = k0 + kk;
-        rb[q] = (n < p.N && k < p.K) ? p.b[(long)k * p.b_sk + (long)n * p.b_sn] : 0.0;
-      }
+      const int m = m0 + idx % GT_M, ka = k0 + idx / GT_M;
+      ra[q] = (m < n && ka < n) ? a[(long)m + (long)ka * n] : 0.0;
+      const int c = n0 + idx / GT_K, kb = k0 + idx % GT_K;
+      rb[q] = (c < n && kb < n) ? b[(long)kb + (long)c * n] : 0.0;
     }
   };
   auto stash = [&]() {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int idx = t + 256 * q;
-      const int kka = (p.a_sk == 1) ? idx % GT_K : idx / GT_M;
-      const int mma = (p.a_sk == 1) ? idx / GT_K : idx % GT_M;
-      As[mma][kka] = ra[q];
-      const int kkb = (p.b_sk == 1) ? idx % GT_K : idx / GT_N;
-      const int nnb = (p.b_sk == 1) ? idx / GT_K : idx % GT_N;
-      Bs[nnb][kkb] = rb[q];
+      As[idx % GT_M][idx / GT_M] = ra[q];
+      Bs[idx / GT_K][idx % GT_K] = rb[q];
     }
   };
-  const bool neg = (p.ep == EP_NEGSUB);
   double acc = 0.0;
   // chunks are staged in a ring of PF register slots, fetched PF chunks
   // ahead of their use, so the global latency overlaps PF chunks of compute
   constexpr int PF = 3;
   double ra_r[PF][4], rb_r[PF][4];
-  const int nchunk = (p.K + GT_K - 1) / GT_K;
+  const int nchunk = (n + GT_K - 1) / GT_K;
   auto fetch_to = [&](int c, double (&ra_)[4], double (&rb_)[4]) {
     fetch(c * GT_K);
 #pragma unroll
@@ -715,7 +702,7 @@ __global__ __launch_bounds__(256) void gemm_square_kernel(GemmArgs p) {
       const int c = c0 + d;
       if (c >= nchunk) break;
       const int k0 = c * GT_K;
-      const int kc = min(GT_K, p.K - k0);
+      const int kc = min(GT_K, n - k0);
       __syncthreads();
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -786,8 +773,16 @@ __global__ __launch_bounds__(256) void gemm_square_kernel(GemmArgs p) {
       }
     }
   }
-  const int n = n0 + tn, m = m0 + tm;
-  if (n < p.N && m < p.M) p.out[(long)m + (long)n * p.out_ld] = acc;
+  const int col = n0 + tn, row = m0 + tm;
+  if (col < n && row < n) out[(long)row + (long)col * n] = acc;
+}
+
+hipError_t launch_square_product(const double *a, const double *b, double *out, int n, bool neg, hipStream_t st) {
+  if (n < 1) return hipErrorInvalidValue;
+  const int ntl = (n + GT_N - 1) / GT_N;
+  hipLaunchKernelGGL(gemm_square_kernel, dim3((unsigned)placed_workgroups(ntl, ntl)), dim3(256), 0, st, a, b, out, n,
+                     neg ? 1 : 0);
+  return hipGetLastError();
 }
 
 // T(i, k) = R(i, k) * CY(k, cyrow): columns of an n x n column-major matrix
@@ -823,8 +818,6 @@ static int gemm_seq_waves(const GemmArgs &a) {
 constexpr int GS_FEW = 8;
 
 long gemm_workgroups(const GemmArgs &a) {
-  if (a.ep == EP_NEGSUB || a.ep == EP_COLMAJ)
-    return 8L * ((a.M + GT_M - 1) / GT_M) * (((a.N + GT_N - 1) / GT_N + 7) / 8);
   if (a.M <= GS_FEW) return (a.N + 3) / 4;
   const int nt = 4 * gemm_seq_waves(a);
   return 8L * ((a.M + 15) / 16) * (((a.N + nt - 1) / nt + 7) / 8);
@@ -845,13 +838,7 @@ static void gemm_few_go(const GemmArgs &a, hipStream_t st, hipEvent_t ev0, hipEv
 }
 
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
-  if (a.M < 1 || a.N < 1 || a.K < 1) return hipErrorInvalidValue;
-  if (a.ep == EP_NEGSUB || a.ep == EP_COLMAJ) {
-    if (a.a_sm != 1 || a.b_sk != 1) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(gemm_square_kernel, dim3((unsigned)gemm_workgroups(a)), dim3(256), 0, st, a);
-    return hipGetLastError();
-  }
-  if (a.a_sk != 1 || a.b_sk != 1 || a.K < 2) return hipErrorInvalidValue;
+  if (a.M < 1 || a.N < 1 || a.K < 2) return hipErrorInvalidValue;
   if (a.M <= GS_FEW) {
     if (a.M == 1) gemm_few_go<1, 12>(a, st, ev0, ev1);
     else if (a.M == 2) gemm_few_go<2, 8>(a, st, ev0, ev1);

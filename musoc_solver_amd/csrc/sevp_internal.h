@@ -155,13 +155,13 @@ struct ResidArgs {  // backward restore + closure residual, one thread per (rhs,
   int apply_row, do_resid;
 };
 
-enum { EP_FWD = 0, EP_BWD = 1, EP_CPL = 2, EP_NEGSUB = 3, EP_COLMAJ = 4 };
+enum { EP_FWD = 0, EP_BWD = 1, EP_CPL = 2 };
 
 struct GemmArgs {  // D(m, n) = sum_k A(m, k) B(k, n), sequential k
-  const double *a;
-  long a_sm, a_sk;
-  const double *b;
-  long b_sk, b_sn;
+  const double *a;    // consecutive k adjacent, rows a_sm apart
+  long a_sm;
+  const double *b;    // consecutive k adjacent, columns b_sn apart
+  long b_sn;
   int M, N, K;
   int ep;
   // EP_FWD / EP_BWD : X row update, per RHS m
@@ -170,7 +170,7 @@ struct GemmArgs {  // D(m, n) = sum_k A(m, k) B(k, n), sequential k
   int xrow;           // 1-based X row updated (ieb for FWD, js+1 for BWD)
   double *dum0;       // EP_FWD: DUM0(:, nb) per RHS
   long dum0_stride;
-  double *out;        // EP_BWD: hfree (M, N); EP_CPL: hcpl (M, N); EP_NEGSUB: (ld out_ld)
+  double *out;        // EP_BWD: hfree (M, N); EP_CPL: hcpl (M, N)
   long out_ld;
   double *g;          // EP_BWD: coupling input g = c * CY(n, cyrow) (may be null)
   const float *cy;
@@ -339,6 +339,8 @@ hipError_t launch_hom_resid(const MarchArgs &m, const ResidArgs *r, hipStream_t 
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t st, hipEvent_t ev0 = nullptr,
                        hipEvent_t ev1 = nullptr);
 long gemm_workgroups(const GemmArgs &a);  // grid size of launch_gemm
+// out = a b, or 0 - a b by successive subtractions (neg): n x n column-major, sequential k
+hipError_t launch_square_product(const double *a, const double *b, double *out, int n, bool neg, hipStream_t st);
 hipError_t launch_cvt_f32(const double *src, float *dst, long n, hipStream_t st);
 // FP32 "lane tiles" of nmat consecutive (K x N) column-major FP64 matrices
 // (the B layout of launch_gemm_part); lane_tiles_floats is one matrix's size.
