@@ -2898,16 +2898,16 @@ extern "C" int sevp_matinv(double *b, int n) {
 
 // ------------------------------------------- MATINV with no allocation
 // A device-pointer MATINV that allocates nothing: the blocked inversion's
-// scratch (panel rows and multipliers, 2 * 32 * n doubles) and the zero-pivot
-// counter live in `scratch`, a file-scope device array of a fixed size, one
-// copy per GPU for the life of the process.  Host code never passes the
+// scratch (two halves each of a panel's rows and columns, 4 * 32 * n doubles) and
+// the zero-pivot counter live in `scratch`, a file-scope device array of a fixed
+// size, one copy per GPU for the life of the process.  Host code never passes the
 // array's name to a kernel (it is a host-side stand-in there): its device
 // address is looked up once per device with hipGetSymbolAddress, with that
 // device current, and that address is what the kernels get.  Calls on one
 // GPU share the array: calls that overlap in time on one GPU race.
 namespace {
 constexpr int kNoAllocMaxN = 4096;
-constexpr size_t kNoAllocCounter = 4 * 32 * (size_t)kNoAllocMaxN;  // counter slot (in doubles)
+constexpr size_t kNoAllocCounter = matinv_blocked_scratch(kNoAllocMaxN, 1);  // counter slot (in doubles)
 constexpr size_t kNoAllocDoubles = kNoAllocCounter + 32;           // 4 MiB + 256 B
 constexpr int kNoAllocDevices = 64;
 std::mutex g_noalloc_mu;

@@ -350,7 +350,10 @@ hipError_t launch_cvt_lane_tiles(const double *src, float *dst, int K, int N, lo
 hipError_t launch_matinv(double *mats, long mat_stride, int n, int count, int *zero_pivots,
                          double *scratch, hipStream_t st);
 bool matinv_uses_lds(int n);
-size_t matinv_blocked_scratch(int n, int count);
+// Pivots per panel of the blocked MATINV, and the doubles of its scratch: two
+// halves each of a panel's rows and columns, per matrix.
+constexpr int MB_KB = 32;
+constexpr size_t matinv_blocked_scratch(int n, int count) { return (size_t)4 * count * MB_KB * n; }
 hipError_t launch_matinv_blocked(double *mats, long ms, int n, int count, int *zp,
                                  double *scratch, hipStream_t st);
 hipError_t launch_scale_cols(const double *r, const float *cy, int cyrow, int i2, double *t,

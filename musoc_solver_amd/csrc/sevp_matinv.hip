@@ -39,8 +39,6 @@
 
 namespace sevp {
 
-constexpr int MB_KB = 32;
-
 #define BM(i, j) B[(long)(i) + (long)(j) * n]  // 0-based, column-major
 
 // Forward panel [p0, p0 + kb).  Workgroups [0, ncol): the panel's steps on 64
@@ -361,11 +359,6 @@ __global__ void mb_copy_rows_kernel(const double *mats, long ms, int n, int kb, 
   if (t < (long)kb * n) rqs[(long)blockIdx.y * qs + (t % kb) * n + t / kb] = BM((int)(t % kb), (int)(t / kb));
 }
 #undef BM
-
-size_t matinv_blocked_scratch(int n, int count) {
-  // Rq and Cq, two halves of KB * n doubles each, per matrix
-  return (size_t)4 * count * MB_KB * n;
-}
 
 hipError_t launch_matinv_blocked(double *mats, long ms, int n, int count, int *zp,
                                  double *scratch, hipStream_t st) {
