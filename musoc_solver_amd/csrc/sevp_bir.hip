@@ -194,7 +194,9 @@ struct Closure {
     if constexpr (WMAX == 32)
       return __hiloint2double(__builtin_amdgcn_ds_bpermute(src, __double2hiint(e)),
                               __builtin_amdgcn_ds_bpermute(src, __double2loint(e)));
+    wave_lds_sync();  // the dot product before has read eb
     eb[lane] = e;
+    wave_lds_sync();
     return e;
   }
   __device__ double dot(double q, const double (&r)[NC]) const {

@@ -82,6 +82,14 @@ __device__ __forceinline__ void unroll(F f) {
   }
 }
 
+// Between LDS writes and reads of the same words by other lanes of the wavefront:
+// the hardware makes a wavefront's LDS operations in order, this keeps the
+// compiler to it.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Broadcast lane `src` (wave-uniform) of a double.
 __device__ __forceinline__ double read_lane(double v, int src) {
   int lo = __builtin_amdgcn_readlane(__double2loint(v), src);

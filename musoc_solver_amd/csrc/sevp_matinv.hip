@@ -180,6 +180,7 @@ __global__ __launch_bounds__(MP_THREADS) void mb_panel_kernel(double *mats, long
 #pragma unroll
     for (int q = 0; q < MB_KB; ++q) Xs[2 * q + h][c] = c < kb ? v[q] : 0.0;
   }
+  wave_lds_sync();
   double y[MB_KB], m[MB_KB], d;
 #pragma unroll
   for (int k = 0; k < MB_KB; ++k) y[k] = Xs[lane][k];
@@ -191,6 +192,7 @@ __global__ __launch_bounds__(MP_THREADS) void mb_panel_kernel(double *mats, long
   panel_cols<24>(y, m, d, 8, colb, Xs[lane]);
   panel_cols<16>(y, m, d, 16, colb, Xs[lane]);
   panel_cols<8>(y, m, d, 24, colb, Xs[lane]);
+  wave_lds_sync();
 #pragma unroll
   for (int q = 0; q < MB_KB; ++q) {
     const int cc = 64 * b + 2 * q + h;
