@@ -802,19 +802,23 @@ hipError_t launch_scale_cols(const double *r, const float *cy, int cyrow, int i2
   return hipGetLastError();
 }
 
-// Computing wavefronts per workgroup of gemm_seq_kernel: as few as leave at
-// most one workgroup per CU, so that every CU streams a share of the matrix
-// and no CU runs two workgroups while another has none.
+// Computing wavefronts per workgroup of gemm_seq_kernel: as few of 1, 2, 4 and 8
+// as leave at most one workgroup per CU, so that no CU runs two workgroups while
+// another has none.  That is 240 of the 256 CUs at 960 columns and 64 right-hand
+// sides, but 180 at 720 x 32, 720 x 64, 1440 x 32 and 1440 x 64, 152 at 1200 x 64
+// and 135 at 1440 x 48 (columns x right-hand sides).
 static int gemm_seq_waves(const GemmArgs &a) {
   const long nmb = (a.M + 15) / 16;
   for (int nw : {1, 2, 4})
     if (nmb * ((a.N + 4 * nw - 1) / (4 * nw)) <= 256) return nw;
   return 8;
 }
-// Right-hand sides up to which the sums are added apart: 8 at 720 columns
-// take 8.7 us that way, 9.5 in gemm_seq_kernel, whose time is the same for
-// any count up to 16; past 8 the forming wavefronts would read more rows than
-// they can keep ahead.
+// Right-hand sides up to which the sums are added apart; past 8 the forming
+// wavefronts would read more rows than they can keep ahead.  gemm_seq_kernel takes
+// the same time for any count up to 16, so 8 against 9 right-hand sides compares
+// the two (a pass of 8 blocks): 173 and 177 us at 360 columns, 241 and 262 at 720,
+// 272 and 306 at 960, 404 and 421 at 1440, but 150 and 142 at 200, 140 and 131 at
+// 130.  One right-hand side: 121 at 200, 191 at 720.
 constexpr int GS_FEW = 8;
 
 long gemm_workgroups(const GemmArgs &a) {
