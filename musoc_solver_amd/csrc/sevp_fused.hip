@@ -29,9 +29,9 @@
 //     the next launch (its workgroups come first), when every column is
 //     complete.
 //
-// The last workgroups of a launch read the next launch's matrices into L2: a
-// launch is a chain of latencies (operands, product, epilogue) with the memory
-// idle for most of it.
+// Where that saves time (warms) the last workgroups of a launch read the next
+// launch's matrices into L2: a launch is a chain of latencies (operands, product,
+// epilogue) with the memory idle for most of it.
 //
 // A pass is 2*NB0 + 1 launches instead of 4*NB0 + 2, each influence matrix is
 // read from HBM once for all right-hand sides, and no partial products go
