@@ -777,13 +777,15 @@ static void rhs_go(const FusedBwdArgs &a, hipStream_t st, hipEvent_t e0, hipEven
 }
 
 // The kernel without the part that brings the next matrices near, for launches
-// of two row tiles that do not: that part's code alone costs them (a pass with 24
+// that do not: that part's code alone costs those of two row tiles (a pass with 24
 // right-hand sides, 16 wavefronts: FP32 64 x 48 271 us without it, 282 with, 200 x
-// 152 929, 977; FP64 800 x 24 224, 234).  The other kernels take as long either way, or are
-// faster with it (FP32, 8 wavefronts, 720 x 40: 1.02 of the time without).
+// 152 929, 977; FP64 800 x 24 224, 234) and the two-per-CU ones, whose registers
+// are full (FP32 1440 x 720, 64, two groups: 31.5 ms a solve, 32.2 with).  The
+// other kernels take as long either way, or are faster with it (FP32, 8
+// wavefronts, two row tiles, 720 x 40: 1.02 of the time without).
 template <class KT, int W, int MBW, bool PICK, class Args>
 static void warm_go(const Args &a, hipStream_t st, hipEvent_t e0, hipEvent_t e1) {
-  if constexpr (MBW == 2 && (W == 16 || std::is_same<KT, KF64>::value))
+  if constexpr (two_per_cu<KT, W, MBW>() || (MBW == 2 && (W == 16 || std::is_same<KT, KF64>::value)))
     if (!a.next) return rhs_go<KT, W, MBW, PICK, false>(a, st, e0, e1);
   rhs_go<KT, W, MBW, PICK, true>(a, st, e0, e1);
 }
