@@ -1797,14 +1797,24 @@ static int ensure_group_streams(sevp_plan p, int groups) {
 // Whether a full-width pass runs on the plan's non-blocking stream, ordered
 // after and before the caller's stream by an event either way.  On a blocking
 // stream every launch made while the null stream has work is made to wait for
-// it, a barrier each: plain FP64 behind work on the null stream, 720 x 360 with
-// one right-hand side (900 launches) 8.5 ms a call there and 5.9 here, 960 x
-// 480 with 64 18.8 and 13.2, 240 x 120 (60 blocks) 1.35 and 1.16.  Below about
-// 32 blocks the host's launches are the longer part and both take the same, so
-// those stay on the caller's stream, as do a non-blocking stream's, a capturing
-// one's (its capture sees only its own launches) and a profiled plan's.
+// it, a barrier each; but a stream that waits for another one slows that one's
+// launches down, by 0.7 us each.  Calls one after another, each behind work on the
+// null stream (and without such work), ms a call there and here:
+//   plain FP64, one right-hand side: 240 x 120 1.39 and 1.15 (1.01, 1.09), 720 x
+//     360 7.5 and 5.6 (4.7, 5.4); 720 x 360, 24 11.3 and 7.9 (7.1, 7.7): here, from
+//     about 32 blocks on; with fewer the host's launches are the longer part
+//   fused, FP32: 240 x 120, one 0.74 and 0.72 (0.53, 0.66), 480 x 240 1.32 and 1.42
+//     (1.16, 1.34); 600 x 300, 8 2.03 and 1.87 (1.58, 1.79), 720 x 360, 24 3.9 and
+//     3.2 (2.9, 3.1), 1440 x 240, 8 2.9 and 2.3 (2.05, 2.2): here, from about 600
+//     columns on, where a launch takes longer than the host's part of it
+//   split K, FP32: 240 x 120, one 0.85 and 0.87 (0.83, 0.84), 720 x 360, 24 3.8 and
+//     3.7 (3.1, 3.7): there
+// So are a non-blocking stream's, a capturing one's (its capture sees only its own
+// launches) and a profiled plan's.
 static bool pass_detours(sevp_plan p, hipStream_t st) {
-  constexpr int kMinBlocks = 32;
+  constexpr int kMinBlocks = 32, kMinFusedColumns = 600;
+  if (p->d.precision != SEVP_PREC_FP64 && (p->pass_kind != SEVP_PASS_FUSED || p->d.i2 < kMinFusedColumns))
+    return false;
   unsigned flags = 0;
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   return p->d.nb0 >= kMinBlocks && p->prof.kclass < 0 &&
